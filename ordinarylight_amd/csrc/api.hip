@@ -391,7 +391,7 @@ int olhip_scene_create(olhip_ctx* ctx, const olhip_scene_desc* d, olhip_scene** 
     }
     BvhInput in{sc->positions.as<float4>(), sc->vidx.as<uint4>(), d->triangle_count, d->leaf_size,
                 boxes.empty() ? nullptr : boxes.data()};
-    bvh_build(in, sc->bvh, s, nullptr, true);
+    bvh_build(in, sc->bvh, s, true);
     upload_faces(sc.get(), d, s);
     build_shade_records(sc->bvh, sc->vidx.as<uint4>(), sc->normals.as<float4>(), d->triangle_count, true, s,
                         d->face_params ? sc->face_orig.as<float4>() : nullptr,
@@ -534,7 +534,7 @@ void build_top_level(olhip_scene* sc, const olhip_instanced_desc* d, hipStream_t
   upload(sc->tlas_vidx, tvidx.data(), tvidx.size(), s);
   OL_HIP_CHECK(hipStreamSynchronize(s));
   BvhInput tin{sc->tlas_pos.as<float4>(), sc->tlas_vidx.as<uint4>(), I, 1u, d->world_bounds, kIsolateLarge};
-  bvh_build(tin, sc->bvh, s, nullptr);
+  bvh_build(tin, sc->bvh, s);
   // The instance table in top-level leaf order: a top-level leaf's first
   // slot is then its instance's index, and entering an instance needs no
   // read of the leaf record.
@@ -645,7 +645,7 @@ int olhip_scene_create_instanced(olhip_ctx* ctx, const olhip_instanced_desc* d, 
         }
         BvhInput in{sc->positions.as<float4>() + vo, sc->vidx.as<uint4>() + to, nt, d->leaf_size,
                     boxes.empty() ? nullptr : boxes.data()};
-        bvh_build(in, *out_r, s, nullptr, true);
+        bvh_build(in, *out_r, s, true);
         build_shade_records(*out_r, sc->vidx.as<uint4>() + to, sc->normals.as<float4>() + vo, nt, false, s);
       }
       blas[r] = BlasDev{out_r->nodes.as<WideNode>(), out_r->tri.as<float4>(), sc->vidx.as<uint4>() + to,
@@ -836,8 +836,7 @@ int olhip_scene_bvh(const olhip_scene* scene, void* nodes, void* tri) {
     require(scene != nullptr, "scene must not be NULL");
     OL_HIP_CHECK(hipSetDevice(scene->ctx->device));
     OL_HIP_CHECK(hipStreamSynchronize(scene->ctx->stream));
-    if (nodes && scene->bvh.node_count)
-      OL_HIP_CHECK(hipMemcpy(nodes, scene->bvh.nodes.ptr, 64ull * scene->bvh.node_count, hipMemcpyDeviceToHost));
+    if (nodes && scene->bvh.node_count) bvh_export_nodes(scene->bvh, static_cast<Node4*>(nodes));
     if (tri && scene->tri_count)
       OL_HIP_CHECK(hipMemcpy(tri, scene->bvh.tri.ptr, 48ull * scene->tri_count, hipMemcpyDeviceToHost));
   });
@@ -859,7 +858,7 @@ int choose_stack(const olhip_ctx* ctx, const olhip_scene* sc) {
 GiLaunch make_launch(olhip_ctx* ctx, const olhip_scene* sc) {
   GiLaunch l{};
   l.cu_count = ctx->cu_count;
-  l.stack_depth = (int)(3u * std::max<uint32_t>(sc->bvh.depth, 1) + 1u);
+  l.stack_depth = (int)(3u * std::max<uint32_t>(sc->bvh.depth, 1) + 2u);
   l.lds_stack = ctx->lds_stack;
   l.trace_block = ctx->trace_block;
   uint64_t words = trace_spill_words(l);
@@ -1210,7 +1209,7 @@ int olhip_trace_device(olhip_ctx* ctx, const olhip_scene* sc, const float* d_ori
     // array; the grid is capped so that its lanes' columns fit there.
     GiLaunch l{};
     l.cu_count = ctx->cu_count;
-    l.stack_depth = (int)(3u * std::max<uint32_t>(sc->bvh.depth, 1) + 1u);
+    l.stack_depth = (int)(3u * std::max<uint32_t>(sc->bvh.depth, 1) + 2u);
     l.lds_stack = ctx->lds_stack;
     l.trace_block = ctx->trace_block;
     l.spill = ctx->trace_scratch;

@@ -1,11 +1,12 @@
 // GPU LBVH build: 30-bit Morton codes -> stable LDS radix sort -> Karras
 // binary radix tree -> bottom-up boxes -> breadth-first collapse into the
-// 64-byte 4-wide node format of common.h.
+// 64-byte 4-wide nodes of common.h that traversal reads.
 //
-// Every step is integer work or exact float min/max/compare, so the result is
-// bit-identical to the sequential CPU build of the same algorithm in
-// oracle/lbvh_oracle.c (checked by tests/test_bvh_gpu.py).  Node numbering is
-// breadth-first with per-level exclusive scans (no atomics decide an index).
+// Every step is integer work or exact float min/max/compare, so the nodes
+// are bit-identical to the sequential CPU build of the same algorithm in
+// oracle/lbvh_oracle.c, up to their numbering: the nodes of a level take
+// their indices from atomics.  Hits do not depend on it, and the exported
+// form (bvh_export_nodes) is renumbered breadth-first.
 //
 // Replaces the driver acceleration-structure builds of the reference
 // (targets/vulkan/scene.py:1132-1194, :1480-1561).
@@ -13,6 +14,7 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
+#include <cstring>
 #include <thread>
 #include <vector>
 
@@ -247,14 +249,16 @@ __device__ __forceinline__ void ref_box(uint32_t ref, const float4* lmin, const 
   }
 }
 
+// Boxes of the triangles in leaf order.
 __global__ void __launch_bounds__(kBlock) k_leaf_boxes(const uint32_t* __restrict__ sorted, uint32_t n,
-                                                       const float4* __restrict__ tmin, const float4* __restrict__ tmax,
+                                                       const float4* __restrict__ pos, const uint4* __restrict__ vidx,
                                                        float4* __restrict__ lmin, float4* __restrict__ lmax) {
-  uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+  const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
   if (k >= n) return;
-  uint32_t o = sorted[k];
-  lmin[k] = tmin[o];
-  lmax[k] = tmax[o];
+  const uint4 t = vidx[sorted[k]];
+  const float4 a = pos[t.x], b = pos[t.y], c = pos[t.z];
+  lmin[k] = make_float4(fminf(fminf(a.x, b.x), c.x), fminf(fminf(a.y, b.y), c.y), fminf(fminf(a.z, b.z), c.z), 0.0f);
+  lmax[k] = make_float4(fmaxf(fmaxf(a.x, b.x), c.x), fmaxf(fmaxf(a.y, b.y), c.y), fmaxf(fmaxf(a.z, b.z), c.z), 0.0f);
 }
 
 __global__ void __launch_bounds__(kBlock) k_bottom_up(uint32_t n, const uint32_t* __restrict__ left,
@@ -281,7 +285,7 @@ __global__ void __launch_bounds__(kBlock) k_bottom_up(uint32_t n, const uint32_t
   }
 }
 
-// ---- 6. breadth-first collapse to 4-wide nodes --------------------------------------------
+// ---- 6. breadth-first collapse to wide nodes -----------------------------------------------
 struct TreeView {
   const uint32_t *left, *right, *rfirst, *rlast;
   const float4 *lmin, *lmax, *bmin, *bmax;
@@ -307,53 +311,8 @@ __device__ __forceinline__ uint32_t ref_count(const TreeView& t, uint32_t ref) {
 __device__ __forceinline__ uint32_t ref_first(const TreeView& t, uint32_t ref) {
   return (ref & OL_LEAF_BIT) ? (ref & ~OL_LEAF_BIT) : t.rfirst[ref];
 }
-__device__ __forceinline__ float ref_area(const TreeView& t, uint32_t ref) {
-  float4 mn, mx;
-  ref_box(ref, t.lmin, t.lmax, t.bmin, t.bmax, mn, mx);
-  float dx = mx.x - mn.x, dy = mx.y - mn.y, dz = mx.z - mn.z;
-  return 2.0f * ((dx * dy + dy * dz) + dz * dx);
-}
 __device__ __forceinline__ bool ref_is_wide_leaf(const TreeView& t, uint32_t ref) {
   return (ref & OL_LEAF_BIT) || ref_count(t, ref) <= t.leaf_size;
-}
-
-// Greedy opening: repeatedly replace the largest-area child that is not a
-// wide leaf by its two children, until four children or nothing to open.
-__device__ int plan_children(const TreeView& t, uint32_t ref, uint32_t kids[4]) {
-  if (ref_is_wide_leaf(t, ref)) {
-    kids[0] = ref;
-    return 1;
-  }
-  int nk = 2;
-  kids[0] = t.left[ref];
-  kids[1] = t.right[ref];
-  while (nk < 4) {
-    int best = -1;
-    float best_area = -1.0f;
-    for (int k = 0; k < nk; ++k) {
-      if (ref_is_wide_leaf(t, kids[k])) continue;
-      float a = ref_area(t, kids[k]);
-      if (a > best_area) { best_area = a; best = k; }
-    }
-    if (best < 0) break;
-    uint32_t r = kids[best];
-    for (int k = nk; k > best + 1; --k) kids[k] = kids[k - 1];
-    kids[best] = t.left[r];
-    kids[best + 1] = t.right[r];
-    ++nk;
-  }
-  return nk;
-}
-
-__global__ void __launch_bounds__(kBlock) k_collapse_plan(TreeView t, const uint32_t* __restrict__ front, uint32_t count,
-                                                          uint32_t* __restrict__ inner_count) {
-  uint32_t k = blockIdx.x * kBlock + threadIdx.x;
-  if (k >= count) return;
-  uint32_t kids[4];
-  int nk = plan_children(t, front[k], kids);
-  uint32_t c = 0;
-  for (int i = 0; i < nk; ++i) c += ref_is_wide_leaf(t, kids[i]) ? 0u : 1u;
-  inner_count[k] = c;
 }
 
 // Quantise one axis of up to four child boxes against the node box [lo, hi].
@@ -383,63 +342,139 @@ OL_HD uint32_t quant_hi(float lo, float scale, float v) {
   return (uint32_t)q;
 }
 
-__global__ void __launch_bounds__(kBlock) k_collapse_emit(TreeView t, const uint32_t* __restrict__ front, uint32_t count,
-                                                          uint32_t level_base, uint32_t next_base,
-                                                          const uint32_t* __restrict__ offsets,
-                                                          uint32_t* __restrict__ next_front, WideNode* __restrict__ nodes) {
-  uint32_t k = blockIdx.x * kBlock + threadIdx.x;
-  if (k >= count) return;
-  uint32_t kids[4];
-  int nk = plan_children(t, front[k], kids);
-  float4 cmn[4], cmx[4];
-  float4 nmn = make_float4(INFINITY, INFINITY, INFINITY, 0.0f), nmx = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
-  const float pad = box_pad(t);
-  for (int i = 0; i < nk; ++i) {
-    ref_box(kids[i], t.lmin, t.lmax, t.bmin, t.bmax, cmn[i], cmx[i]);
-    cmn[i] = make_float4(cmn[i].x - pad, cmn[i].y - pad, cmn[i].z - pad, 0.0f);
-    cmx[i] = make_float4(cmx[i].x + pad, cmx[i].y + pad, cmx[i].z + pad, 0.0f);
-    nmn = make_float4(fminf(nmn.x, cmn[i].x), fminf(nmn.y, cmn[i].y), fminf(nmn.z, cmn[i].z), 0.0f);
-    nmx = make_float4(fmaxf(nmx.x, cmx[i].x), fmaxf(nmx.y, cmx[i].y), fmaxf(nmx.z, cmx[i].z), 0.0f);
-  }
-  WideNode node;
-  node.ox = nmn.x;
-  node.oy = nmn.y;
-  node.oz = nmn.z;
-  uint32_t ex = quant_exponent(nmn.x, nmx.x), ey = quant_exponent(nmn.y, nmx.y), ez = quant_exponent(nmn.z, nmx.z);
-  node.exps = ex | (ey << 8) | (ez << 16);
-  float sx = exp_scale(ex), sy = exp_scale(ey), sz = exp_scale(ez);
-  uint32_t qlo[3] = {0, 0, 0}, qhi[3] = {0, 0, 0};
-  uint32_t r = 0;
-  for (int i = 0; i < 4; ++i) {
-    if (i >= nk) {
-      node.child[i] = OL_NONE;
-      continue;
-    }
-    qlo[0] |= quant_lo(nmn.x, sx, cmn[i].x) << (8 * i);
-    qlo[1] |= quant_lo(nmn.y, sy, cmn[i].y) << (8 * i);
-    qlo[2] |= quant_lo(nmn.z, sz, cmn[i].z) << (8 * i);
-    qhi[0] |= quant_hi(nmn.x, sx, cmx[i].x) << (8 * i);
-    qhi[1] |= quant_hi(nmn.y, sy, cmx[i].y) << (8 * i);
-    qhi[2] |= quant_hi(nmn.z, sz, cmx[i].z) << (8 * i);
-    uint32_t ref = kids[i];
-    if (ref_is_wide_leaf(t, ref)) {
-      node.child[i] = OL_LEAF_BIT | ((ref_count(t, ref) - 1u) << 27) | ref_first(t, ref);
-    } else {
-      uint32_t slot = offsets[k] + r++;
-      node.child[i] = next_base + slot;
-      next_front[slot] = ref;
-    }
-  }
-  for (int a = 0; a < 3; ++a) {
-    node.qlo[a] = qlo[a];
-    node.qhi[a] = qhi[a];
-  }
-  node.pad[0] = 0;
-  node.pad[1] = 0;
-  nodes[level_base + k] = node;
+// One level of the wide nodes: four lanes per node, one per child.
+//
+// Greedy opening: the child of largest area that is not a leaf (the first in
+// leaf order of several) is replaced by its two children, until there are
+// four; the two lanes concerned load their boxes.  Children take their slots
+// in leaf order, and their lanes write their bytes of the planes; places in
+// the next level come from one atomic per wave.  Levels run one after the other on
+// the stream, each reading its size from device memory, so the host looks at
+// the sizes only every kNodeLevels levels.
+constexpr uint32_t kNodeLevels = 12;
+constexpr uint32_t W_WORDS = kNodeLevels + 1;  // sizes of the queued levels and of the next
+
+__global__ void k_nodes_begin(uint32_t* ctr, uint32_t* front, uint32_t root) {
+  const uint32_t t = threadIdx.x;
+  if (t < W_WORDS) ctr[t] = t == 0u ? 1u : 0u;
+  if (t == 0u) front[0] = root;
+}
+// The size of the level after the queued ones becomes the first.
+__global__ void k_nodes_next(uint32_t* ctr) {
+  const uint32_t n = ctr[kNodeLevels];
+  __syncthreads();
+  if (threadIdx.x <= kNodeLevels) ctr[threadIdx.x] = threadIdx.x == 0u ? n : 0u;
 }
 
-// ---- 7. leaf-order traversal triangles ----------------------------------------------------------
+// `before`: nodes of the levels before the queued ones.  The level's nodes
+// follow those of the levels before it, in the order of its list.
+__global__ void __launch_bounds__(kBlock) k_nodes_level(TreeView t, const uint32_t* __restrict__ front,
+                                                        uint32_t* __restrict__ next, uint32_t* ctr, uint32_t level,
+                                                        uint32_t before, WideNode* __restrict__ nodes) {
+  const uint32_t n = ctr[level];
+  uint32_t base = before;
+  for (uint32_t l = 0; l < level; ++l) base += ctr[l];
+  const uint32_t lane = lane_id(), j = lane & 3u, head = lane & ~3u;
+  const uint32_t waves = gridDim.x * (kBlock / 64u);
+  const float pad = n ? box_pad(t) : 0.0f;
+  for (uint32_t first = (blockIdx.x * (kBlock / 64u) + threadIdx.x / 64u) * 16u; first < n; first += waves * 16u) {
+    const uint32_t item = first + (lane >> 2);
+    const bool valid = item < n;
+    const uint32_t root = valid ? front[item] : 0u;
+    // This lane's child: `ref` (has: there is one), its box, and its area
+    // (negative when it is a leaf or there is none).
+    uint32_t ref = 0, pos = OL_NONE, nk = 0;
+    bool has = false;
+    float area = -1.0f;
+    float4 mn = make_float4(INFINITY, INFINITY, INFINITY, 0.0f), mx = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
+    auto set = [&](uint32_t r) {
+      ref = r;
+      has = true;
+      pos = ref_first(t, r);
+      ref_box(r, t.lmin, t.lmax, t.bmin, t.bmax, mn, mx);
+      const float dx = mx.x - mn.x, dy = mx.y - mn.y, dz = mx.z - mn.z;
+      const float a = 2.0f * ((dx * dy + dy * dz) + dz * dx);
+      area = ref_is_wide_leaf(t, r) ? -1.0f : (a >= 0.0f ? a : 3.0e38f);
+    };
+    if (valid) {
+      if (ref_is_wide_leaf(t, root)) {
+        if (j == 0u) set(root);
+        nk = 1;
+      } else {
+        if (j < 2u) set(j ? t.right[root] : t.left[root]);
+        nk = 2;
+      }
+    }
+    for (int round = 0; round < 2; ++round) {
+      float a = area;
+      uint32_t who = j, at = pos;
+      for (uint32_t off = 1; off < 4u; off <<= 1) {
+        const float oa = __shfl_xor(a, (int)off, 64);
+        const uint32_t ow = (uint32_t)__shfl_xor((int)who, (int)off, 64), op = (uint32_t)__shfl_xor((int)at, (int)off, 64);
+        if (oa > a || (oa == a && op < at)) {
+          a = oa;
+          who = ow;
+          at = op;
+        }
+      }
+      const uint32_t r = (uint32_t)__shfl((int)ref, (int)(head | who), 64);
+      if (a >= 0.0f && nk >= 2u) {
+        if (j == who) set(t.left[r]);
+        else if (j == nk) set(t.right[r]);
+        ++nk;
+      }
+    }
+    const bool inner = has && area >= 0.0f;
+    const float3 lo = make_float3(mn.x - pad, mn.y - pad, mn.z - pad), hi = make_float3(mx.x + pad, mx.y + pad, mx.z + pad);
+    float3 nlo = lo, nhi = hi;
+    for (uint32_t off = 1; off < 4u; off <<= 1) {
+      nlo.x = fminf(nlo.x, __shfl_xor(nlo.x, (int)off, 64));
+      nlo.y = fminf(nlo.y, __shfl_xor(nlo.y, (int)off, 64));
+      nlo.z = fminf(nlo.z, __shfl_xor(nlo.z, (int)off, 64));
+      nhi.x = fmaxf(nhi.x, __shfl_xor(nhi.x, (int)off, 64));
+      nhi.y = fmaxf(nhi.y, __shfl_xor(nhi.y, (int)off, 64));
+      nhi.z = fmaxf(nhi.z, __shfl_xor(nhi.z, (int)off, 64));
+    }
+    // Slot: the child's rank in leaf order (lanes without one come last).
+    uint32_t slot = 0;
+    for (uint32_t off = 1; off < 4u; ++off) {
+      const uint32_t other = head | ((j + off) & 3u);
+      const uint32_t op = (uint32_t)__shfl((int)pos, (int)other, 64);
+      slot += (op < pos || (op == pos && other < lane)) ? 1u : 0u;
+    }
+    // Places of the inner children in the next level.
+    const uint64_t inners = __ballot(inner);
+    uint32_t at = 0;
+    if (lane == 0u && inners) at = atomicAdd(&ctr[level + 1u], (uint32_t)__popcll(inners));
+    const uint32_t place = (uint32_t)__shfl((int)at, 0, 64) + lanes_below(inners);
+    if (inner) next[place] = ref;
+    if (!valid) continue;
+    WideNode* node = nodes + (base + item);
+    const float sx = exp_scale(quant_exponent(nlo.x, nhi.x)), sy = exp_scale(quant_exponent(nlo.y, nhi.y)),
+                sz = exp_scale(quant_exponent(nlo.z, nhi.z));
+    if (j == 0u) {
+      node->ox = nlo.x;
+      node->oy = nlo.y;
+      node->oz = nlo.z;
+      node->sx = sx;
+      node->sy = sy;
+      node->sz = sz;
+    }
+    uint8_t* ql = reinterpret_cast<uint8_t*>(node->qlo) + slot;
+    uint8_t* qh = reinterpret_cast<uint8_t*>(node->qhi) + slot;
+    ql[0] = has ? (uint8_t)quant_lo(nlo.x, sx, lo.x) : 255;
+    ql[4] = has ? (uint8_t)quant_lo(nlo.y, sy, lo.y) : 255;
+    ql[8] = has ? (uint8_t)quant_lo(nlo.z, sz, lo.z) : 255;
+    qh[0] = has ? (uint8_t)quant_hi(nlo.x, sx, hi.x) : 0;
+    qh[4] = has ? (uint8_t)quant_hi(nlo.y, sy, hi.y) : 0;
+    qh[8] = has ? (uint8_t)quant_hi(nlo.z, sz, hi.z) : 0;
+    node->child[slot] = !has ? OL_LEAF_BIT
+                        : inner ? base + n + place
+                                : OL_LEAF_BIT | ((ref_count(t, ref) - 1u) << 27) | ref_first(t, ref);
+  }
+}
+
+// ---- 7. traversal triangles in leaf order ---------------------------------------------------------
 __global__ void __launch_bounds__(kBlock) k_reorder(const uint32_t* __restrict__ sorted, uint32_t n,
                                                     const float4* __restrict__ pos, const uint4* __restrict__ vidx,
                                                     float4* __restrict__ tri) {
@@ -459,95 +494,115 @@ inline dim3 grid_for(uint32_t n) { return dim3((n + kBlock - 1) / kBlock); }
 
 namespace {
 
-// Boxes of every leaf and binary node for the current vertex positions, the
-// wide collapse, and the leaf-order triangles (steps 5-7 of the build).
-void build_boxes(const BvhInput& in, const BvhTopology& tp, BvhOutput& out, hipStream_t s, BvhDebug* debug) {
-  const uint32_t n = in.tri_count;
-  const uint32_t leaf_size = tp.leaf_size;
-  DevBuf tmin, tmax, cb;
-  tmin.reserve(sizeof(float4) * n);
-  tmax.reserve(sizeof(float4) * n);
-  cb.reserve(sizeof(int) * 8);
-  hipLaunchKernelGGL(k_init_bounds, dim3(1), dim3(64), 0, s, cb.as<int>());
-  hipLaunchKernelGGL(k_tri_bounds, grid_for(n), dim3(kBlock), 0, s, in.positions, in.tri_vidx, n, tmin.as<float4>(),
-                     tmax.as<float4>(), cb.as<int>());
-  const uint32_t ni = n > 1 ? n - 1 : 1;
+// Boxes of every leaf and binary node of a topology for the current vertex
+// positions (step 5).
+struct TreeBoxes {
   DevBuf lmin, lmax, bmin, bmax, flags;
-  lmin.reserve(sizeof(float4) * n);
-  lmax.reserve(sizeof(float4) * n);
-  bmin.reserve(sizeof(float4) * ni);
-  bmax.reserve(sizeof(float4) * ni);
-  flags.reserve(4ull * ni);
-  hipLaunchKernelGGL(k_leaf_boxes, grid_for(n), dim3(kBlock), 0, s, tp.sorted.as<uint32_t>(), n, tmin.as<float4>(),
-                     tmax.as<float4>(), lmin.as<float4>(), lmax.as<float4>());
+};
+
+TreeView compute_boxes(const BvhInput& in, const BvhTopology& tp, TreeBoxes& b, uint32_t leaf_size, hipStream_t s) {
+  const uint32_t n = in.tri_count, ni = n > 1 ? n - 1 : 1;
+  b.lmin.reserve(sizeof(float4) * n);
+  b.lmax.reserve(sizeof(float4) * n);
+  b.bmin.reserve(sizeof(float4) * ni);
+  b.bmax.reserve(sizeof(float4) * ni);
+  b.flags.reserve(4ull * ni);
+  hipLaunchKernelGGL(k_leaf_boxes, grid_for(n), dim3(kBlock), 0, s, tp.sorted.as<uint32_t>(), n, in.positions,
+                     in.tri_vidx, b.lmin.as<float4>(), b.lmax.as<float4>());
   if (n > 1) {
-    OL_HIP_CHECK(hipMemsetAsync(flags.ptr, 0, 4ull * ni, s));
+    OL_HIP_CHECK(hipMemsetAsync(b.flags.ptr, 0, 4ull * ni, s));
     hipLaunchKernelGGL(k_bottom_up, grid_for(n), dim3(kBlock), 0, s, n, tp.left.as<uint32_t>(),
                        tp.right.as<uint32_t>(), tp.parent_int.as<uint32_t>(), tp.parent_leaf.as<uint32_t>(),
-                       lmin.as<float4>(), lmax.as<float4>(), bmin.as<float4>(), bmax.as<float4>(),
-                       flags.as<uint32_t>());
+                       b.lmin.as<float4>(), b.lmax.as<float4>(), b.bmin.as<float4>(), b.bmax.as<float4>(),
+                       b.flags.as<uint32_t>());
   }
-  if (debug) {
-    OL_HIP_CHECK(hipStreamSynchronize(s));
-    debug->sorted_index.resize(n);
-    OL_HIP_CHECK(hipMemcpy(debug->sorted_index.data(), tp.sorted.ptr, 4ull * n, hipMemcpyDeviceToHost));
-    if (n > 1) {
-      debug->left.resize(n - 1);
-      debug->right.resize(n - 1);
-      debug->node_box.resize(8ull * (n - 1));
-      OL_HIP_CHECK(hipMemcpy(debug->left.data(), tp.left.ptr, 4ull * (n - 1), hipMemcpyDeviceToHost));
-      OL_HIP_CHECK(hipMemcpy(debug->right.data(), tp.right.ptr, 4ull * (n - 1), hipMemcpyDeviceToHost));
-      std::vector<float4> a(n - 1), b(n - 1);
-      OL_HIP_CHECK(hipMemcpy(a.data(), bmin.ptr, sizeof(float4) * (n - 1), hipMemcpyDeviceToHost));
-      OL_HIP_CHECK(hipMemcpy(b.data(), bmax.ptr, sizeof(float4) * (n - 1), hipMemcpyDeviceToHost));
-      for (uint32_t i = 0; i + 1 < n; ++i) {
-        float* d = &debug->node_box[8ull * i];
-        d[0] = a[i].x; d[1] = a[i].y; d[2] = a[i].z; d[3] = a[i].w;
-        d[4] = b[i].x; d[5] = b[i].y; d[6] = b[i].z; d[7] = b[i].w;
-      }
-    }
-  }
+  return TreeView{tp.left.as<uint32_t>(), tp.right.as<uint32_t>(), tp.rfirst.as<uint32_t>(), tp.rlast.as<uint32_t>(),
+                  b.lmin.as<float4>(), b.lmax.as<float4>(), b.bmin.as<float4>(), b.bmax.as<float4>(), leaf_size,
+                  n > 1 ? 0u : OL_LEAF_BIT};
+}
 
-  // Wide collapse, one breadth-first level per iteration.
-  TreeView tv{tp.left.as<uint32_t>(), tp.right.as<uint32_t>(), tp.rfirst.as<uint32_t>(), tp.rlast.as<uint32_t>(),
-              lmin.as<float4>(), lmax.as<float4>(), bmin.as<float4>(), bmax.as<float4>(), leaf_size,
-              n > 1 ? 0u : OL_LEAF_BIT};
+// The traversal nodes and triangles for the current vertex positions
+// (steps 5-7 of the build).
+void build_nodes(const BvhInput& in, const BvhTopology& tp, BvhOutput& out, hipStream_t s) {
+  const uint32_t n = in.tri_count;
+  TreeBoxes boxes;
+  const TreeView tv = compute_boxes(in, tp, boxes, tp.leaf_size, s);
   out.nodes.reserve(sizeof(WideNode) * (size_t)(n + 1));
-  DevBuf front_a, front_b, icount;
+  out.tri.reserve(sizeof(float4) * 3ull * n);
+  DevBuf front_a, front_b, ctr;
   front_a.reserve(4ull * (n + 1));
   front_b.reserve(4ull * (n + 1));
-  icount.reserve(4ull * (n + 2));
-  uint32_t root = n > 1 ? 0u : OL_LEAF_BIT;
-  OL_HIP_CHECK(hipMemcpyAsync(front_a.ptr, &root, 4, hipMemcpyHostToDevice, s));
-  uint32_t level_count = 1, level_base = 0, depth = 0;
-  uint32_t* cur = front_a.as<uint32_t>();
-  uint32_t* nxt = front_b.as<uint32_t>();
-  while (level_count > 0) {
-    ++depth;
-    hipLaunchKernelGGL(k_collapse_plan, grid_for(level_count), dim3(kBlock), 0, s, tv, cur, level_count,
-                       icount.as<uint32_t>());
-    scan_exclusive_u32(icount.as<uint32_t>(), level_count, icount.as<uint32_t>() + level_count, s);
-    uint32_t next_count = 0;
-    OL_HIP_CHECK(hipMemcpyAsync(&next_count, icount.as<uint32_t>() + level_count, 4, hipMemcpyDeviceToHost, s));
+  ctr.reserve(4ull * W_WORDS);
+  uint32_t *cur = front_a.as<uint32_t>(), *nxt = front_b.as<uint32_t>();
+  hipLaunchKernelGGL(k_nodes_begin, dim3(1), dim3(64), 0, s, ctr.as<uint32_t>(), cur, tv.root);
+  uint32_t words[W_WORDS];
+  uint64_t bound = 1;  // nodes of the level at most
+  out.depth = 0;
+  out.node_count = 0;
+  while (true) {
+    for (uint32_t l = 0; l < kNodeLevels; ++l) {
+      const uint64_t blocks = (std::min<uint64_t>(bound, n) * 4 + kBlock - 1) / kBlock;
+      hipLaunchKernelGGL(k_nodes_level, dim3((unsigned)std::min<uint64_t>(blocks, 4096)), dim3(kBlock), 0, s, tv, cur,
+                         nxt, ctr.as<uint32_t>(), l, out.node_count, out.nodes.as<WideNode>());
+      std::swap(cur, nxt);
+      if (bound < n) bound *= 4;
+    }
+    OL_HIP_CHECK(hipMemcpyAsync(words, ctr.ptr, sizeof(words), hipMemcpyDeviceToHost, s));
     OL_HIP_CHECK(hipStreamSynchronize(s));
-    uint32_t next_base = level_base + level_count;
-    hipLaunchKernelGGL(k_collapse_emit, grid_for(level_count), dim3(kBlock), 0, s, tv, cur, level_count, level_base,
-                       next_base, icount.as<uint32_t>(), nxt, out.nodes.as<WideNode>());
-    level_base = next_base;
-    level_count = next_count;
-    std::swap(cur, nxt);
+    for (uint32_t l = 0; l < kNodeLevels && words[l]; ++l) {
+      ++out.depth;
+      out.node_count += words[l];
+    }
+    if (words[kNodeLevels] == 0u) break;
+    hipLaunchKernelGGL(k_nodes_next, dim3(1), dim3(64), 0, s, ctr.as<uint32_t>());
   }
-  out.node_count = level_base;
-  out.depth = depth;
-
-  out.tri.reserve(sizeof(float4) * 3ull * n);
-  hipLaunchKernelGGL(k_reorder, grid_for(n), dim3(kBlock), 0, s, tp.sorted.as<uint32_t>(), n, in.positions,
-                     in.tri_vidx, out.tri.as<float4>());
+  hipLaunchKernelGGL(k_reorder, grid_for(n), dim3(kBlock), 0, s, tp.sorted.as<uint32_t>(), n, in.positions, in.tri_vidx,
+                     out.tri.as<float4>());
   OL_HIP_CHECK(hipGetLastError());
   OL_HIP_CHECK(hipStreamSynchronize(s));
 }
 
 }  // namespace
+
+void bvh_export_nodes(const BvhOutput& built, Node4* out) {
+  const uint32_t n = built.node_count;
+  std::vector<WideNode> nodes(n);
+  if (n == 0) return;
+  OL_HIP_CHECK(hipMemcpy(nodes.data(), built.nodes.ptr, sizeof(WideNode) * (size_t)n, hipMemcpyDeviceToHost));
+  auto exponent = [](float scale) {
+    uint32_t bits;
+    std::memcpy(&bits, &scale, sizeof(bits));
+    return bits >> 23;
+  };
+  std::vector<uint32_t> order{0u};  // breadth-first: place -> built index
+  order.reserve(n);
+  for (uint32_t k = 0; k < order.size(); ++k) {
+    const WideNode& w = nodes[order[k]];
+    Node4 o{};
+    o.ox = w.ox;
+    o.oy = w.oy;
+    o.oz = w.oz;
+    o.exps = exponent(w.sx) | (exponent(w.sy) << 8) | (exponent(w.sz) << 16);
+    for (uint32_t c = 0; c < 4u; ++c) {
+      const uint32_t byte = 255u << (8u * c);
+      if ((w.qlo[0] & byte) > (w.qhi[0] & byte)) {  // inverted: no child
+        o.child[c] = OL_NONE;
+        continue;
+      }
+      for (int a = 0; a < 3; ++a) {
+        o.qlo[a] |= w.qlo[a] & byte;
+        o.qhi[a] |= w.qhi[a] & byte;
+      }
+      if (child_is_leaf(w.child[c])) {
+        o.child[c] = w.child[c];
+      } else {
+        o.child[c] = (uint32_t)order.size();
+        order.push_back(w.child[c]);
+      }
+    }
+    out[k] = o;
+  }
+}
 
 // Binned SAH over primitive boxes, one primitive per leaf: a top-down split
 // of [b, e) at the best of 16 centroid bins on each axis (surface area x
@@ -726,14 +781,14 @@ void upload_vec(DevBuf& d, const std::vector<T>& v, hipStream_t s) {
 
 }  // namespace
 
-void bvh_build(const BvhInput& in, BvhOutput& out, hipStream_t s, BvhDebug* debug, bool keep_topology) {
+void bvh_build(const BvhInput& in, BvhOutput& out, hipStream_t s, bool keep_topology) {
   auto t0 = std::chrono::steady_clock::now();
   const uint32_t n = in.tri_count;
   out.topology.reset();
   if (n == 0) {
     out.node_count = 0;
     out.depth = 0;
-    out.nodes.reserve(64);
+    out.nodes.reserve(sizeof(WideNode));
     out.tri.reserve(48);
     return;
   }
@@ -752,7 +807,7 @@ void bvh_build(const BvhInput& in, BvhOutput& out, hipStream_t s, BvhDebug* debu
     upload_vec(tp->parent_int, pi, s);
     upload_vec(tp->parent_leaf, pl, s);
     OL_HIP_CHECK(hipStreamSynchronize(s));
-    build_boxes(in, *tp, out, s, debug);
+    build_nodes(in, *tp, out, s);
     if (keep_topology) out.topology = std::move(tp);
     out.build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return;
@@ -772,11 +827,6 @@ void bvh_build(const BvhInput& in, BvhOutput& out, hipStream_t s, BvhDebug* debu
                      tmax.as<float4>(), cb.as<int>());
   hipLaunchKernelGGL(k_morton, grid_for(n), dim3(kBlock), 0, s, tmin.as<float4>(), tmax.as<float4>(), n, cb.as<int>(),
                      codes.as<uint32_t>(), tp->sorted.as<uint32_t>());
-  if (debug) {
-    OL_HIP_CHECK(hipStreamSynchronize(s));
-    debug->morton.resize(n);
-    OL_HIP_CHECK(hipMemcpy(debug->morton.data(), codes.ptr, sizeof(uint32_t) * n, hipMemcpyDeviceToHost));
-  }
   radix_sort_pairs(codes.as<uint32_t>(), tp->sorted.as<uint32_t>(), codes_tmp.as<uint32_t>(),
                    vals_tmp.as<uint32_t>(), n, s, 32);
   codes_tmp.release();
@@ -795,7 +845,7 @@ void bvh_build(const BvhInput& in, BvhOutput& out, hipStream_t s, BvhDebug* debu
                        tp->left.as<uint32_t>(), tp->right.as<uint32_t>(), tp->rfirst.as<uint32_t>(),
                        tp->rlast.as<uint32_t>(), tp->parent_int.as<uint32_t>(), tp->parent_leaf.as<uint32_t>());
   // Steps 5-7.
-  build_boxes(in, *tp, out, s, debug);
+  build_nodes(in, *tp, out, s);
   if (keep_topology) out.topology = std::move(tp);
   out.build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
@@ -806,6 +856,6 @@ void bvh_refit(const BvhInput& in, BvhOutput& out, hipStream_t s) {
   if (!out.topology) throw OlError{-1, "the BVH was built without a kept topology"};
   const BvhTopology& tp = *out.topology;
   if (tp.tri_count != in.tri_count) throw OlError{-1, "refit needs the triangle count of the build"};
-  build_boxes(in, tp, out, s, nullptr);
+  build_nodes(in, tp, out, s);
   out.build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }

@@ -176,10 +176,31 @@ OL_DEV uint32_t wave_reserve_n(uint32_t* counter, uint32_t n) {
 }
 
 // -- scene records ---------------------------------------------------------------
-// 4-wide BVH node, 64 bytes (one cache-line-aligned record, four dwordx4 loads).
-// Child boxes are 8-bit offsets from `origin` in units of 2^(e-127) per axis,
-// rounded outward at build time against the exact float decode below.
+// 4-wide BVH node, 64 bytes: four dwordx4 loads, each lane its own node.
+// The vector L1 serves one such 16-byte load per clock and CU, so a node's
+// bytes cost as much as its arithmetic (128-byte nodes of eight children
+// visited a quarter fewer nodes and were 25-45 % slower).
+//
+// Child boxes are 8-bit offsets from the origin in units of a power of two
+// per axis, rounded outward at build time against the float decode; the
+// units are stored as floats, ready to use.  A missing child has an inverted
+// box and the word of a leaf holding triangle (or instance) 0: where
+// rounding lets a far ray meet that box all the same, it tests a triangle
+// that is part of the scene, which cannot change a result, so no child word
+// needs a validity test.
 struct alignas(64) WideNode {
+  float ox, oy, oz, sx;
+  uint32_t qlo[3];    // byte c = child c, per axis x/y/z
+  float sy;
+  uint32_t qhi[3];
+  float sz;
+  uint32_t child[4];  // leaf: OL_LEAF_BIT | (count-1) << 27 | first, or inner index
+};
+static_assert(sizeof(WideNode) == 64, "WideNode must be 64 bytes");
+
+// The form that olhip_scene_bvh copies out: numbered breadth-first, packed
+// exponents, missing children marked.
+struct alignas(64) Node4 {
   float ox, oy, oz;
   uint32_t exps;      // ex | ey << 8 | ez << 16 (biased by 127)
   uint32_t qlo[3];    // byte c = child c, per axis x/y/z
@@ -187,7 +208,7 @@ struct alignas(64) WideNode {
   uint32_t child[4];  // OL_NONE | leaf: 0x80000000 | (count-1) << 27 | first | inner index
   uint32_t pad[2];
 };
-static_assert(sizeof(WideNode) == 64, "WideNode must be 64 bytes");
+static_assert(sizeof(Node4) == 64, "Node4 must be 64 bytes");
 
 constexpr uint32_t OL_LEAF_BIT = 0x80000000u;
 constexpr uint32_t OL_LEAF_MAX = 16u;

@@ -201,16 +201,19 @@ __global__ void __launch_bounds__(BLOCK) k_e0_trace(E0Params P, E0State S, uint3
       while (true) {
         uint4 w0, w1, w2, w3;
         load_node(P.sc.nodes, node, w0, w1, w2, w3);
-        uint32_t ch[4], key[4];
-        node_children(w2, w3, ch);
         const float cull = bt < (U)3.0e38 ? cull_distance((float)bt) + 1e-6f : INFINITY;
-        ol_node_keys(w0, w1, w2, rp, 0.0f, cull, key, ch);
+        double p[4];
+        const uint32_t hits = node_children<true>(w0, w1, w2, w3, rp, 0.0f, cull, p);
+        // Near to far (the last hit child first): leaves are tested at once,
+        // the nearest inner child comes next, the others go on the stack.
         uint32_t next = OL_NONE;
-        for (int c = 0; c < 4; ++c) {
-          if (key[c] == OL_NONE) continue;
-          if (child_is_leaf(ch[c])) {
-            for (uint32_t k = 0; k < leaf_count(ch[c]); ++k) {
-              const uint32_t slot = leaf_first(ch[c]) + k;
+#pragma unroll
+        for (int k = 3; k >= 0; --k) {
+          if ((uint32_t)k >= hits) continue;
+          const uint32_t c = pair_word(p[k]);
+          if (child_is_leaf(c)) {
+            for (uint32_t j2 = 0; j2 < leaf_count(c); ++j2) {
+              const uint32_t slot = leaf_first(c) + j2;
               const float4 a = P.sc.tri[3 * slot], e1 = P.sc.tri[3 * slot + 1], e2 = P.sc.tri[3 * slot + 2];
               E0Hit<OT, DT> h = e0_tri<OT, DT>(o, d, a, e1, e2);
               const uint32_t orig = __float_as_uint(a.w);
@@ -220,9 +223,9 @@ __global__ void __launch_bounds__(BLOCK) k_e0_trace(E0Params P, E0State S, uint3
               }
             }
           } else if (next == OL_NONE) {
-            next = ch[c];
+            next = c;
           } else if (sp < (uint32_t)STACK) {
-            col[(sp++) * BLOCK] = ch[c];
+            col[(sp++) * BLOCK] = c;
           } else {
             atomicOr(&S.ctr[1], 1u);
           }

@@ -214,7 +214,7 @@ GiLaunch Engine::make_launch() {
   quiesce();
   GiLaunch l{};
   l.cu_count = ctx_->cu_count;
-  l.stack_depth = (int)(3u * (uint32_t)std::max(max_depth_, 1) + 1u);
+  l.stack_depth = (int)(3u * (uint32_t)std::max(max_depth_, 1) + 2u);
   l.lds_stack = cfg_.lds_stack;
   l.trace_block = cfg_.trace_block;
   const uint64_t words = trace_spill_words(l);

@@ -183,7 +183,7 @@ struct Wave {
 // Traversal launch shape.
 struct GiLaunch {
   int cu_count;
-  int stack_depth;   // total traversal stack entries needed (3 * BVH depth + 1)
+  int stack_depth;   // total traversal stack entries needed (3 * BVH depth + 2)
   int lds_stack;     // entries kept in LDS: 8, 12, 16, 24, 32, 48
   int trace_block;   // 64, 128, 256
   uint32_t* spill;   // global spill columns for entries beyond lds_stack

@@ -1658,12 +1658,9 @@ k_primary(Wave W, uint32_t in, uint32_t* spill, uint32_t spill_cap) {
       rd = mk4(dir, 1e30f);
       hv = make_float4(rd.w, 0.0f, 0.0f, __uint_as_float(OL_NONE));
       if (sc.node_count != 0u) {
-        ClosestRay q;
-        closest_begin(q, mk3(ro), mk3(rd), ro.w, rd.w);
-        st.sp = 0;
-        while (!closest_step<LSTACK>(sc.nodes, sc.tri, q, st, nv, nt)) {
-        }
-        hv = make_float4(q.best.t, q.best.u, q.best.v, __uint_as_float(q.best.slot));
+        const TraceHit h = ol_trace_closest<LSTACK>(sc.nodes, sc.tri, sc.node_count, mk3(ro), mk3(rd), ro.w, rd.w, st,
+                                                    nv, nt);
+        hv = make_float4(h.t, h.u, h.v, __uint_as_float(h.slot));
       }
     }
     shade_chunk<kFull>(W, in, 1u, k, path, ro, rd, hv);
@@ -1828,7 +1825,7 @@ void launch_rays(const GiLaunch& l, const DScene& sc, const float4* o, const flo
 }  // namespace
 
 int stack_depth_for(uint32_t bvh_depth) {
-  uint32_t need = 3u * bvh_depth + 1u;
+  const uint32_t need = 3u * bvh_depth + 2u;
   const int depths[] = {16, 24, 32, 48, 64, 96, 128};
   for (int d : depths)
     if ((uint32_t)d >= need) return d;

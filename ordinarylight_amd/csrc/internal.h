@@ -111,14 +111,6 @@ struct BvhOutput {
   std::unique_ptr<BvhTopology> topology;  // kept when the build asked for it (refit)
 };
 
-// Optional debug capture of intermediate build arrays (bit-exact checks).
-struct BvhDebug {
-  std::vector<uint32_t> morton;       // [T] per original triangle
-  std::vector<uint32_t> sorted_index; // [T] original index of sorted position
-  std::vector<uint32_t> left, right;  // [T-1] binary children (leaf refs | 0x80000000)
-  std::vector<float> node_box;        // [T-1][8] binary internal boxes (min.xyzw, max.xyzw)
-};
-
 // Host binned-SAH binary hierarchy over n >= 2 primitive boxes (min xyz, max
 // xyz each), one primitive per leaf, in the Karras arrays' conventions: leaf
 // order, children (leaf refs | OL_LEAF_BIT), leaf ranges, parents.  isolate:
@@ -128,7 +120,10 @@ void sah_topology(const float* box, uint32_t n, std::vector<uint32_t>& order, st
                   std::vector<uint32_t>& parent_int, std::vector<uint32_t>& parent_leaf, bool isolate = false);
 
 // keep_topology: retain the binary topology in out.topology for bvh_refit.
-void bvh_build(const BvhInput& in, BvhOutput& out, hipStream_t stream, BvhDebug* debug, bool keep_topology = false);
+void bvh_build(const BvhInput& in, BvhOutput& out, hipStream_t stream, bool keep_topology = false);
+// The built nodes in their exported form: numbered breadth-first, exponents
+// packed, missing children marked (node_count records).
+void bvh_export_nodes(const BvhOutput& built, Node4* out);
 // Recomputes the boxes, the wide nodes and the leaf triangles of a kept
 // topology for new vertex positions (same triangles, same indices), as an
 // acceleration-structure update does: the leaf order stays, boxes follow the

@@ -4,8 +4,8 @@
 // LSTACK entries live in LDS, one column per lane (entry k of lane t at
 // lds[k * BLOCK + t], bank-conflict free), deeper entries spill to a per-lane
 // column of a global buffer.  The total depth is chosen on the host from the
-// BVH's level count (a 4-wide level pushes at most three entries), so it
-// cannot overflow; the small LDS part keeps occupancy bounded by registers,
+// BVH's level count (a 4-wide level leaves at most three entries, and four
+// are pushed before the next is taken), so it cannot overflow; the small LDS part keeps occupancy bounded by registers,
 // not LDS.
 //
 // Closest-hit semantics are those of a ray query over opaque triangles
@@ -72,10 +72,35 @@ OL_DEV RayPre ray_pre_fast(f3 o, f3 d) {
 
 OL_DEV float byte_f(uint32_t w, int c) { return (float)((w >> (8 * c)) & 255u); }
 
+// a where the bits of m are clear, b where they are set: one v_bitop3_b32,
+// which issues twice as fast as a v_cndmask_b32 and needs no compare.
+OL_DEV uint32_t bit_select(uint32_t a, uint32_t b, uint32_t m) { return __builtin_amdgcn_bitop3_b32(a, b, m, 0xD8); }
+// a | (b & c)
+OL_DEV uint32_t or_and(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0xF8); }
+
+// A child of a node as one 64-bit number: its sort key above its child word.
+// Keys are non-negative floats, or have the sign bit set for a missed child,
+// so as doubles the pairs order by key with misses last (no pair is a NaN or
+// an infinity: the top bits are those of a float, whose exponent field ends
+// two bits lower).  v_min_f64 and v_max_f64 exchange a pair in two
+// instructions at the issue rate of their float32 forms, where comparing
+// keys and moving keys and words took a compare and four selects.
+OL_DEV double child_pair(uint32_t key, uint32_t word) {
+  return __builtin_bit_cast(double, (uint64_t)key << 32 | word);
+}
+OL_DEV uint32_t pair_word(double p) { return (uint32_t)__builtin_bit_cast(uint64_t, p); }
+OL_DEV void pair_order(double& a, double& b) {
+  double hi, lo;
+  asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+  asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+  a = hi;
+  b = lo;
+}
+
 // Slab test of the four quantised child boxes of a node.
 //
-// Plane q of axis a lies at origin_a + q * 2^e_a; its ray distance is taken
-// as fma(q, 2^e_a * inv_a, (origin_a - o_a) * inv_a), three float32 roundings
+// Plane q of axis a lies at origin_a + q * s_a; its ray distance is taken as
+// fma(q, s_a * inv_a, (origin_a - o_a) * inv_a), three float32 roundings
 // of quantities no larger than the scene extent plus the origin distance.
 // The near plane of each axis is the low plane when the direction is
 // positive and the high plane otherwise, so each child costs six fma and
@@ -83,62 +108,40 @@ OL_DEV float byte_f(uint32_t w, int c) { return (float)((w >> (8 * c)) & 255u); 
 // scene coordinate, far more (in space) than these roundings, so a box that
 // contains a candidate hit is never culled.
 //
-// Returns one sort key per child: the entry distance's bits with the low two
-// bits replaced by the child's position, or OL_NONE when the child is empty
-// or missed.  Entry distances are >= tmin >= 0, so unsigned key order is
-// distance order.
-OL_DEV void ol_node_keys(const uint4 w0, const uint4 w1, const uint4 w2, const RayPre& r, float tmin, float tmax,
-                         uint32_t key[4], const uint32_t child[4]) {
-  const float ax = exp_scale(w0.w & 255u) * r.inv.x, bx = (__uint_as_float(w0.x) - r.o.x) * r.inv.x;
-  const float ay = exp_scale((w0.w >> 8) & 255u) * r.inv.y, by = (__uint_as_float(w0.y) - r.o.y) * r.inv.y;
-  const float az = exp_scale((w0.w >> 16) & 255u) * r.inv.z, bz = (__uint_as_float(w0.z) - r.o.z) * r.inv.z;
-  const uint32_t nx = (r.neg & 1u) ? w1.w : w1.x, fx = (r.neg & 1u) ? w1.x : w1.w;
-  const uint32_t ny = (r.neg & 2u) ? w2.x : w1.y, fy = (r.neg & 2u) ? w1.y : w2.x;
-  const uint32_t nz = (r.neg & 4u) ? w2.y : w1.z, fz = (r.neg & 4u) ? w1.z : w2.y;
-  const float t0 = fmaxf(tmin, 0.0f);
+// Returns the children as pairs in descending order: hit children from far
+// to near (kNear) or from the last slot to the first, then the missed ones;
+// and the number of hit children.  A child is missed when tf - tn is
+// negative; that sign goes into the key as it is.
+template <bool kNear>
+OL_DEV uint32_t node_children(const uint4 w0, const uint4 w1, const uint4 w2, const uint4 w3, const RayPre& r,
+                              float tmin, float tmax, double p[4]) {
+  const float ax = __uint_as_float(w0.w) * r.inv.x, bx = (__uint_as_float(w0.x) - r.o.x) * r.inv.x;
+  const float ay = __uint_as_float(w1.w) * r.inv.y, by = (__uint_as_float(w0.y) - r.o.y) * r.inv.y;
+  const float az = __uint_as_float(w2.w) * r.inv.z, bz = (__uint_as_float(w0.z) - r.o.z) * r.inv.z;
+  const uint32_t mx = (uint32_t)(__float_as_int(r.inv.x) >> 31), my = (uint32_t)(__float_as_int(r.inv.y) >> 31),
+                 mz = (uint32_t)(__float_as_int(r.inv.z) >> 31);
+  const uint32_t nx = bit_select(w1.x, w2.x, mx), fx = bit_select(w2.x, w1.x, mx);
+  const uint32_t ny = bit_select(w1.y, w2.y, my), fy = bit_select(w2.y, w1.y, my);
+  const uint32_t nz = bit_select(w1.z, w2.z, mz), fz = bit_select(w2.z, w1.z, mz);
+  const uint32_t word[4] = {w3.x, w3.y, w3.z, w3.w};
+  uint32_t hits = 4u;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const float tnx = __builtin_fmaf(byte_f(nx, c), ax, bx), tfx = __builtin_fmaf(byte_f(fx, c), ax, bx);
     const float tny = __builtin_fmaf(byte_f(ny, c), ay, by), tfy = __builtin_fmaf(byte_f(fy, c), ay, by);
     const float tnz = __builtin_fmaf(byte_f(nz, c), az, bz), tfz = __builtin_fmaf(byte_f(fz, c), az, bz);
-    const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, t0));
-    const float tf = fminf(fminf(tfx, tfy), fminf(tfz, tmax));
-    const bool hit = child[c] != OL_NONE && tn <= tf;
-    key[c] = hit ? ((__float_as_uint(tn) & ~3u) | (uint32_t)c) : OL_NONE;
+    const float tn = fmaxf(fmaxf(fmaxf(fmaxf(tnx, tny), tnz), tmin), 0.0f);
+    const float tf = fminf(fminf(fminf(tfx, tfy), tfz), tmax);
+    const uint32_t d = __float_as_uint(tf - tn);
+    p[c] = child_pair(or_and(kNear ? __float_as_uint(tn) : (uint32_t)c, d, 0x80000000u), word[c]);
+    hits += (uint32_t)((int)d >> 31);
   }
-}
-
-OL_DEV void key_swap(uint32_t& a, uint32_t& b) {
-  const uint32_t lo = min(a, b), hi = max(a, b);
-  a = lo;
-  b = hi;
-}
-// Ascending sort of four keys (five compare-exchanges).
-OL_DEV void sort4(uint32_t k[4]) {
-  key_swap(k[0], k[1]);
-  key_swap(k[2], k[3]);
-  key_swap(k[0], k[2]);
-  key_swap(k[1], k[3]);
-  key_swap(k[1], k[2]);
-}
-OL_DEV float key_distance(uint32_t key) { return __uint_as_float(key & ~3u); }
-
-// Ascending sort of four keys carrying their child words along (five
-// compare-exchanges of pairs), so no child needs selecting by key afterwards.
-OL_DEV void pair_swap(uint32_t& ka, uint32_t& kb, uint32_t& ca, uint32_t& cb) {
-  const bool s = kb < ka;
-  const uint32_t k0 = s ? kb : ka, k1 = s ? ka : kb, c0 = s ? cb : ca, c1 = s ? ca : cb;
-  ka = k0;
-  kb = k1;
-  ca = c0;
-  cb = c1;
-}
-OL_DEV void sort4_pairs(uint32_t k[4], uint32_t c[4]) {
-  pair_swap(k[0], k[1], c[0], c[1]);
-  pair_swap(k[2], k[3], c[2], c[3]);
-  pair_swap(k[0], k[2], c[0], c[2]);
-  pair_swap(k[1], k[3], c[1], c[3]);
-  pair_swap(k[1], k[2], c[1], c[2]);
+  pair_order(p[0], p[1]);
+  pair_order(p[2], p[3]);
+  pair_order(p[0], p[2]);
+  pair_order(p[1], p[3]);
+  pair_order(p[1], p[2]);
+  return hits;
 }
 
 // Culling distance for a current best hit at t: boxes entered beyond it are
@@ -195,22 +198,21 @@ struct TravStack {
     }
     ++sp;
   }
-  // Pushes m (0..3) entries: c3 (m = 3), c2 (m >= 2), c1 (m >= 1), in that
-  // order, so c1 ends on top.  When three entries fit in LDS the lane
-  // writes three words unconditionally (those above the new top are
-  // scratch) instead of branching per entry.
-  OL_DEV void push_upto3(uint32_t c1, uint32_t c2, uint32_t c3, uint32_t m) {
-    if (sp + 3u <= (uint32_t)LSTACK) {
-      const uint32_t v0 = m >= 3u ? c3 : (m == 2u ? c2 : c1);
-      const uint32_t v1 = m >= 3u ? c2 : c1;
-      lds[sp * lds_stride] = v0;
-      lds[(sp + 1u) * lds_stride] = v1;
-      lds[(sp + 2u) * lds_stride] = c1;
+  // Pushes the words of the first m (0..4) of p.  Where four entries fit in
+  // LDS the lane writes four words (those above the new top are scratch)
+  // without selecting or branching per entry.
+  OL_DEV void push_pairs(const double p[4], uint32_t m) {
+    if (sp + 4u <= (uint32_t)LSTACK) {
+      lds[sp * lds_stride] = pair_word(p[0]);
+      lds[(sp + 1u) * lds_stride] = pair_word(p[1]);
+      lds[(sp + 2u) * lds_stride] = pair_word(p[2]);
+      lds[(sp + 3u) * lds_stride] = pair_word(p[3]);
       sp += m;
     } else {
-      if (m >= 3u) push(c3);
-      if (m >= 2u) push(c2);
-      if (m >= 1u) push(c1);
+      if (m >= 1u) push(pair_word(p[0]));
+      if (m >= 2u) push(pair_word(p[1]));
+      if (m >= 3u) push(pair_word(p[2]));
+      if (m >= 4u) push(pair_word(p[3]));
     }
   }
   OL_DEV uint32_t pop() {
@@ -225,20 +227,12 @@ struct TravStack {
   OL_DEV void set_bottom(uint32_t v) { lds[0] = v; }
 };
 
-// Children of a node in child-word order.
-OL_DEV void node_children(const uint4 w2, const uint4 w3, uint32_t ch[4]) {
-  ch[0] = w2.z;
-  ch[1] = w2.w;
-  ch[2] = w3.x;
-  ch[3] = w3.y;
-}
-
 // Closest-hit traversal state of one lane, advanced one node per step.
 struct ClosestRay {
   RayPre r;
   float tmin;
   TraceHit best;
-  uint32_t node;  // next node to visit
+  uint32_t node;  // next item to visit
 };
 
 OL_DEV void closest_begin(ClosestRay& q, f3 o, f3 d, float tmin, float tmax) {
@@ -248,84 +242,12 @@ OL_DEV void closest_begin(ClosestRay& q, f3 o, f3 d, float tmin, float tmax) {
   q.node = 0;
 }
 
-// Visits q.node: tests its leaf children (near to far), continues with the
-// nearest inner child and pushes the others far to near, dropping those
-// that start beyond the culling distance.  Returns true when the traversal
-// has finished (nothing left to visit).  nv / nt count nodes visited and
-// triangles tested (work counters).
+// Pushes a node's hit children, the one to visit first on top, and takes
+// the next stack entry (OL_NONE when nothing is left).
 template <int LSTACK>
-OL_DEV bool closest_step(const WideNode* __restrict__ nodes, const float4* __restrict__ tri, ClosestRay& q,
-                         TravStack<LSTACK>& st, uint32_t& nv, uint32_t& nt) {
-  uint4 w0, w1, w2, w3;
-  load_node(nodes, q.node, w0, w1, w2, w3);
-  ++nv;
-  uint32_t ch[4], key[4];
-  node_children(w2, w3, ch);
-  // Cull against the current best distance widened like the slab test.
-  ol_node_keys(w0, w1, w2, q.r, q.tmin, cull_distance(q.best.t), key, ch);
-  sort4(key);
-  // The lexicographic minimum does not depend on the order; nearer leaves
-  // shrink the culling distance sooner.
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (key[k] == OL_NONE) continue;
-    const uint32_t c = ch[key[k] & 3u];
-    if (!child_is_leaf(c)) continue;
-    const uint32_t first = leaf_first(c), cnt = leaf_count(c);
-    nt += cnt;
-    for (uint32_t j = 0; j < cnt; ++j) {
-      const uint32_t slot = first + j;
-      float4 a, e1, e2;
-      load_tri(tri, slot, a, e1, e2);
-      float t, u, v;
-      if (ol_tri_test(q.r.o, q.r.d, a, e1, e2, t, u, v) && t >= q.tmin) {
-        const uint32_t orig = __float_as_uint(a.w);
-        if (t < q.best.t || (t == q.best.t && orig < q.best.orig)) q.best = TraceHit{t, u, v, slot, orig};
-      }
-    }
-  }
-  const float cull = cull_distance(q.best.t);
-  uint32_t next = OL_NONE;
-#pragma unroll
-  for (int k = 3; k >= 0; --k) {
-    if (key[k] == OL_NONE) continue;
-    const uint32_t c = ch[key[k] & 3u];
-    if (child_is_leaf(c) || key_distance(key[k]) > cull) continue;
-    if (next != OL_NONE) st.push(next);
-    next = c;
-  }
-  if (next != OL_NONE) {
-    q.node = next;
-    return false;
-  }
-  if (st.empty()) return true;
-  q.node = st.pop();
-  return false;
-}
-
-// Any hit ends at the first occluder found, so its children need no
-// distance order: they are taken in build order (the first hit child
-// continues), which has measured faster for shadow rays than near to far.
-// The keys become the hit children's positions, ascending, misses last.
-OL_DEV void build_order(uint32_t key[4], uint32_t ch[4]) {
-#pragma unroll
-  for (int k = 0; k < 4; ++k) key[k] = key[k] == OL_NONE ? OL_NONE : (uint32_t)k;
-  sort4_pairs(key, ch);
-}
-
-// With the hit children first and in visiting order, keys and child words
-// sorted together (sort4_pairs or build_order): continues with the first
-// and pushes the others in reverse, so the second is on top; with no child
-// hit, takes the next stack entry.
-template <int LSTACK>
-OL_DEV void descend(TravStack<LSTACK>& st, const uint32_t ch[4], const uint32_t key[4], uint32_t& node) {
-  if (key[0] == OL_NONE) {
-    node = st.empty() ? OL_NONE : st.pop();
-    return;
-  }
-  const uint32_t m = (key[1] != OL_NONE ? 1u : 0u) + (key[2] != OL_NONE ? 1u : 0u) + (key[3] != OL_NONE ? 1u : 0u);
-  st.push_upto3(ch[1], ch[2], ch[3], m);
-  node = ch[0];
+OL_DEV void descend(TravStack<LSTACK>& st, const double p[4], uint32_t hits, uint32_t& node) {
+  st.push_pairs(p, hits);
+  node = st.empty() ? OL_NONE : st.pop();
 }
 
 // Split-step form used by the refilling scheduler.  q.node holds the next
@@ -339,18 +261,16 @@ OL_DEV bool item_is_leaf(uint32_t item) { return child_is_leaf(item); }
 template <int LSTACK>
 OL_DEV void closest_next(ClosestRay& q, TravStack<LSTACK>& st) { q.node = st.empty() ? OL_NONE : st.pop(); }
 
-// Inner step: continue with the nearest hit child (inner or leaf) and push the
-// others far to near.
+// Inner step: continue with the nearest hit child (inner or leaf), the others
+// on the stack.
 template <int LSTACK>
 OL_DEV void closest_inner(const WideNode* __restrict__ nodes, ClosestRay& q, TravStack<LSTACK>& st, uint32_t& nv) {
   uint4 w0, w1, w2, w3;
   load_node(nodes, q.node, w0, w1, w2, w3);
   ++nv;
-  uint32_t ch[4], key[4];
-  node_children(w2, w3, ch);
-  ol_node_keys(w0, w1, w2, q.r, q.tmin, cull_distance(q.best.t), key, ch);
-  sort4_pairs(key, ch);
-  descend(st, ch, key, q.node);
+  double p[4];
+  const uint32_t hits = node_children<true>(w0, w1, w2, w3, q.r, q.tmin, cull_distance(q.best.t), p);
+  descend(st, p, hits, q.node);
 }
 
 // Leaf step: test the leaf's triangles, then take the next stack entry.
@@ -371,8 +291,10 @@ OL_DEV void closest_leaf(const float4* __restrict__ tri, ClosestRay& q, TravStac
   closest_next(q, st);
 }
 
-// Any-hit traversal state of one lane in split-step form (see above).
-// q.node is OL_NONE once finished; occluded tells whether a triangle in
+// Any-hit traversal state of one lane in split-step form (see above).  Any
+// hit ends at the first occluder found, so its children need no distance
+// order: they are taken in slot order, which has measured faster for shadow
+// rays than near to far.  q.node is OL_NONE once finished; occluded tells whether a triangle in
 // [tmin, tmax] was found.
 struct AnyRay {
   RayPre r;
@@ -398,11 +320,9 @@ OL_DEV void any_inner(const WideNode* __restrict__ nodes, AnyRay& q, TravStack<L
   uint4 w0, w1, w2, w3;
   load_node(nodes, q.node, w0, w1, w2, w3);
   ++nv;
-  uint32_t ch[4], key[4];
-  node_children(w2, w3, ch);
-  ol_node_keys(w0, w1, w2, q.r, q.tmin, q.tcull, key, ch);
-  build_order(key, ch);
-  descend(st, ch, key, q.node);
+  double p[4];
+  const uint32_t hits = node_children<false>(w0, w1, w2, w3, q.r, q.tmin, q.tcull, p);
+  descend(st, p, hits, q.node);
 }
 
 template <int LSTACK>
@@ -432,7 +352,9 @@ OL_DEV TraceHit ol_trace_closest(const WideNode* __restrict__ nodes, const float
   closest_begin(q, o, d, tmin, tmax);
   if (node_count == 0) return q.best;
   st.sp = 0;
-  while (!closest_step<LSTACK>(nodes, tri, q, st, nv, nt)) {
+  while (q.node != OL_NONE) {
+    while (!child_is_leaf(q.node) && q.node != OL_NONE) closest_inner<LSTACK>(nodes, q, st, nv);
+    while (child_is_leaf(q.node)) closest_leaf<LSTACK>(tri, q, st, nt);
   }
   return q.best;
 }
@@ -605,11 +527,9 @@ OL_DEV void closest2_node(const DScene& sc, Closest2& q, TravStack<LSTACK>& st, 
   uint4 w0, w1, w2, w3;
   load_node(nodes, q.node, w0, w1, w2, w3);
   ++nv;
-  uint32_t ch[4], key[4];
-  node_children(w2, w3, ch);
-  ol_node_keys(w0, w1, w2, q.r, q.tmin, cull_distance(q.best.t), key, ch);
-  sort4_pairs(key, ch);
-  descend(st, ch, key, q.node);
+  double p[4];
+  const uint32_t hits = node_children<true>(w0, w1, w2, w3, q.r, q.tmin, cull_distance(q.best.t), p);
+  descend(st, p, hits, q.node);
 }
 
 // Entry or node step, whichever the lane is at.
@@ -702,11 +622,9 @@ OL_DEV void any2_node(const DScene& sc, Any2& q, TravStack<LSTACK>& st, uint32_t
   uint4 w0, w1, w2, w3;
   load_node(nodes, q.node, w0, w1, w2, w3);
   ++nv;
-  uint32_t ch[4], key[4];
-  node_children(w2, w3, ch);
-  ol_node_keys(w0, w1, w2, q.r, q.tmin, q.tcull, key, ch);
-  build_order(key, ch);
-  descend(st, ch, key, q.node);
+  double p[4];
+  const uint32_t hits = node_children<false>(w0, w1, w2, w3, q.r, q.tmin, q.tcull, p);
+  descend(st, p, hits, q.node);
 }
 
 template <int LSTACK>
