@@ -110,6 +110,9 @@ OL_DEV uint32_t lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdg
 OL_DEV uint32_t lanes_below(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
+// Lanes whose predicate holds: the compare's mask itself (__ballot takes an
+// int, which costs a select and a second compare).
+OL_DEV uint64_t lanes_where(bool want) { return __builtin_amdgcn_ballot_w64(want); }
 // Reserve one slot per lane whose `want` is true with one atomic per wave.
 // Must be reached by every active lane of the wave.
 OL_DEV uint32_t wave_reserve(uint32_t* counter, bool want) {

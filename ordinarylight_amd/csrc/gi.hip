@@ -414,54 +414,65 @@ OL_DEV void closest_pass(const Wave& W, uint32_t in, TravStack<LSTACK>& st) {
   q.node = OL_NONE;
   const WideNode* nodes = nullptr;
   const float4* tri = nullptr;
-  uint32_t slot = OL_NONE;
-  bool busy = false;
+  uint32_t slot = OL_NONE;  // the lane's ray, until its hit is written
   uint32_t nv = 0, nt = 0;
   while (true) {
-    const uint64_t idle = __ballot(!busy);
-    const uint32_t n_idle = (uint32_t)__popcll(idle);
-    if (n_idle >= kRefillMin) {
+    uint64_t inner = lanes_where(item_is_inner(q.node)), leafy = lanes_where(item_is_leaf(q.node));
+    bool more = !(pool.exhausted && pool.n == 0);
+    if (more && (uint32_t)__popcll(inner | leafy) + kRefillMin <= 64u) {
+      // Finished lanes write their hits and take new rays.
+      if (q.node == OL_NONE && slot != OL_NONE) {
+        W.hit[slot] = make_float4(q.best.t, q.best.u, q.best.v, __uint_as_float(q.best.slot));
+        slot = OL_NONE;
+      }
       pool_refill(pool, W, prefix, top, counts, cursor, c_begin, c_end);
-      const uint32_t take = min(n_idle, pool.n);
-      if (!busy) {
-        const uint32_t rank = lanes_below(idle);
-        if (rank < take) {
-          slot = pool.slot + rank;
-          const float4 o = qo[slot], d = qd[slot];
+      const uint64_t idle = ~(inner | leafy);
+      const uint32_t take = min((uint32_t)__popcll(idle), pool.n);
+      const uint32_t rank = lanes_below(idle);
+      if (q.node == OL_NONE && rank < take) {
+        const uint32_t i = pool.slot + rank;
+        const float4 o = qo[i], d = qd[i];
+        if (pool.node_count == 0) {
+          W.hit[i] = make_float4(d.w, 0.0f, 0.0f, __uint_as_float(OL_NONE));
+        } else {
           closest_begin(q, mk3(o), mk3(d), o.w, d.w);
-          if (pool.node_count == 0) {
-            W.hit[slot] = make_float4(d.w, 0.0f, 0.0f, __uint_as_float(OL_NONE));
-          } else {
-            nodes = pool.nodes;
-            tri = pool.tri;
-            st.sp = 0;
-            busy = true;
-          }
+          slot = i;
+          nodes = pool.nodes;
+          tri = pool.tri;
+          st.sp = 0;
         }
       }
       pool.slot += take;
       pool.n -= take;
+      more = !(pool.exhausted && pool.n == 0);
+      inner = lanes_where(item_is_inner(q.node));
+      leafy = lanes_where(item_is_leaf(q.node));
     }
-    const bool at_leaf = busy && item_is_leaf(q.node);
-    const uint64_t leafy = __ballot(at_leaf);
-    const uint64_t inner = __ballot(busy && !at_leaf);
-    if ((leafy | inner) == 0) {
-      if (pool.exhausted && pool.n == 0) break;
+    if ((inner | leafy) == 0) {
+      if (!more) break;
       continue;
     }
-    if (inner == 0 || 3u * (uint32_t)__popcll(leafy) >= (uint32_t)__popcll(leafy | inner)) {
-      if (at_leaf) closest_leaf<LSTACK>(tri, q, st, nt);
-    } else if (busy && !at_leaf) {
-      closest_inner<LSTACK>(nodes, q, st, nv);
+    // Inner steps until leaves hold a third of the busy lanes, or enough
+    // lanes have finished to take new rays.  A loop of its own keeps the
+    // hit's registers out of it (they are copied where the two kinds of step
+    // meet).
+    uint32_t n_busy = (uint32_t)__popcll(inner | leafy);
+    while (inner != 0 && 3u * (uint32_t)__popcll(leafy) < n_busy) {
+      nv += (uint32_t)__popcll(inner);
+      if (item_is_inner(q.node)) closest_inner<LSTACK>(nodes, q, st);
+      inner = lanes_where(item_is_inner(q.node));
+      leafy = lanes_where(item_is_leaf(q.node));
+      n_busy = (uint32_t)__popcll(inner | leafy);
+      if (more && n_busy + kRefillMin <= 64u) break;
     }
-    if (busy && q.node == OL_NONE) {
-      W.hit[slot] = make_float4(q.best.t, q.best.u, q.best.v, __uint_as_float(q.best.slot));
-      busy = false;
+    if (leafy != 0 && 3u * (uint32_t)__popcll(leafy) >= n_busy) {
+      if (item_is_leaf(q.node)) closest_leaf<LSTACK>(tri, q, st, nt);
     }
   }
-  if (W.work && (nv | nt)) {
-    atomicAdd(&W.work[0], (unsigned long long)nv);
-    atomicAdd(&W.work[1], (unsigned long long)nt);
+  if (slot != OL_NONE) W.hit[slot] = make_float4(q.best.t, q.best.u, q.best.v, __uint_as_float(q.best.slot));
+  if (W.work) {
+    if (nv && lane_id() == 0u) atomicAdd(&W.work[0], (unsigned long long)nv);
+    if (nt) atomicAdd(&W.work[1], (unsigned long long)nt);
   }
 }
 
@@ -507,74 +518,84 @@ OL_DEV void shadow_pass(const Wave& W, uint32_t in, TravStack<LSTACK>& st) {
   q.occluded = false;
   const WideNode* nodes = nullptr;
   const float4* tri = nullptr;
-  uint32_t g = 0, e = 0, e_end = 0, mode = 0;
+  uint32_t g = OL_NONE, e = 0, e_end = 0, mode = 0;  // the lane's group until it is resolved
   f3 direct = mk3(0.0f, 0.0f, 0.0f), area_direct = direct, env_direct = direct;
-  bool busy = false;
   uint32_t nv = 0, nt = 0;
   while (true) {
-    const uint64_t idle = __ballot(!busy);
-    const uint32_t n_idle = (uint32_t)__popcll(idle);
-    if (n_idle >= kRefillMin) {
+    uint64_t inner = lanes_where(item_is_inner(q.node)), leafy = lanes_where(item_is_leaf(q.node));
+    bool more = !(pool.exhausted && pool.n == 0);
+    uint64_t ended = lanes_where(q.node == OL_NONE && g != OL_NONE);
+    if ((more || ended != 0) && (uint32_t)__popcll(inner | leafy) + kRefillMin <= 64u) {
+      // Lanes at the end of an entry go on with their group's next one or
+      // resolve the group; idle lanes take new groups.
+      if (q.node == OL_NONE && g != OL_NONE) {
+        if (!q.occluded) shadow_add(mode, W.ec[e], direct, area_direct, env_direct);
+        ++e;
+        if (e < e_end) {
+          const float4 o = W.eo[e], d = W.ed[e];
+          any_begin(q, mk3(o), mk3(d), o.w, d.w);
+          st.sp = 0;
+        } else {
+          shadow_resolve(W, g, direct, area_direct, env_direct);
+          g = OL_NONE;
+        }
+      }
       pool_refill(pool, W, prefix, top, counts, cursor, c_begin, c_end);
-      const uint32_t take = min(n_idle, pool.n);
-      if (!busy) {
-        const uint32_t rank = lanes_below(idle);
-        if (rank < take) {
-          g = pool.slot + rank;
-          const uint4 gI = W.gI[g];
-          e = gI.y;
-          e_end = gI.y + gI.z;
-          mode = gI.w >> 16;
-          direct = mk3(0.0f, 0.0f, 0.0f);
-          area_direct = direct;
-          env_direct = direct;
-          if (pool.node_count == 0) {
-            // Nothing can occlude: every entry is visible.
-            for (; e < e_end; ++e) shadow_add(mode, W.ec[e], direct, area_direct, env_direct);
-            shadow_resolve(W, g, direct, area_direct, env_direct);
-          } else if (e < e_end) {
-            const float4 o = W.eo[e], d = W.ed[e];
-            any_begin(q, mk3(o), mk3(d), o.w, d.w);
-            nodes = pool.nodes;
-            tri = pool.tri;
-            st.sp = 0;
-            busy = true;
-          } else {
-            shadow_resolve(W, g, direct, area_direct, env_direct);
-          }
+      const uint64_t idle = lanes_where(q.node == OL_NONE);
+      const uint32_t take = min((uint32_t)__popcll(idle), pool.n);
+      const uint32_t rank = lanes_below(idle);
+      if (q.node == OL_NONE && rank < take) {
+        g = pool.slot + rank;
+        const uint4 gI = W.gI[g];
+        e = gI.y;
+        e_end = gI.y + gI.z;
+        mode = gI.w >> 16;
+        direct = mk3(0.0f, 0.0f, 0.0f);
+        area_direct = direct;
+        env_direct = direct;
+        if (pool.node_count != 0 && e < e_end) {
+          const float4 o = W.eo[e], d = W.ed[e];
+          any_begin(q, mk3(o), mk3(d), o.w, d.w);
+          nodes = pool.nodes;
+          tri = pool.tri;
+          st.sp = 0;
+        } else {
+          // Nothing can occlude: every entry is visible.
+          for (; e < e_end; ++e) shadow_add(mode, W.ec[e], direct, area_direct, env_direct);
+          shadow_resolve(W, g, direct, area_direct, env_direct);
+          g = OL_NONE;
         }
       }
       pool.slot += take;
       pool.n -= take;
+      more = !(pool.exhausted && pool.n == 0);
+      inner = lanes_where(item_is_inner(q.node));
+      leafy = lanes_where(item_is_leaf(q.node));
+      ended = 0;
     }
-    const bool at_leaf = busy && item_is_leaf(q.node);
-    const uint64_t leafy = __ballot(at_leaf);
-    const uint64_t inner = __ballot(busy && !at_leaf);
-    if ((leafy | inner) == 0) {
-      if (pool.exhausted && pool.n == 0) break;
+    if ((inner | leafy) == 0) {
+      if (!more && ended == 0) break;
       continue;
     }
-    if (inner == 0 || 3u * (uint32_t)__popcll(leafy) >= (uint32_t)__popcll(leafy | inner)) {
-      if (at_leaf) any_leaf<LSTACK>(tri, q, st, nt);
-    } else if (busy && !at_leaf) {
-      any_inner<LSTACK>(nodes, q, st, nv);
+    uint32_t n_busy = (uint32_t)__popcll(inner | leafy);
+    while (inner != 0 && 3u * (uint32_t)__popcll(leafy) < n_busy) {
+      nv += (uint32_t)__popcll(inner);
+      if (item_is_inner(q.node)) any_inner<LSTACK>(nodes, q, st);
+      inner = lanes_where(item_is_inner(q.node));
+      leafy = lanes_where(item_is_leaf(q.node));
+      const uint32_t left = (uint32_t)__popcll(inner | leafy);
+      // Lanes that ended in this loop may have another entry to trace.
+      const bool refill = left != n_busy && left + kRefillMin <= 64u;
+      n_busy = left;
+      if (refill) break;
     }
-    if (busy && q.node == OL_NONE) {
-      if (!q.occluded) shadow_add(mode, W.ec[e], direct, area_direct, env_direct);
-      ++e;
-      if (e < e_end) {
-        const float4 o = W.eo[e], d = W.ed[e];
-        any_begin(q, mk3(o), mk3(d), o.w, d.w);
-        st.sp = 0;
-      } else {
-        shadow_resolve(W, g, direct, area_direct, env_direct);
-        busy = false;
-      }
+    if (leafy != 0 && 3u * (uint32_t)__popcll(leafy) >= n_busy) {
+      if (item_is_leaf(q.node)) any_leaf<LSTACK>(tri, q, st, nt);
     }
   }
-  if (W.work && (nv | nt)) {
-    atomicAdd(&W.work[2], (unsigned long long)nv);
-    atomicAdd(&W.work[3], (unsigned long long)nt);
+  if (W.work) {
+    if (nv && lane_id() == 0u) atomicAdd(&W.work[2], (unsigned long long)nv);
+    if (nt) atomicAdd(&W.work[3], (unsigned long long)nt);
   }
 }
 
@@ -619,66 +640,81 @@ OL_DEV void closest2_pass(const Wave& W, uint32_t in, TravStack<LSTACK>& st) {
   Closest2 q;
   q.node = OL_NONE;
   q.inst = OL_NONE;
-  uint32_t job = 0, slot = OL_NONE;
-  bool busy = false;
+  uint32_t job = 0, slot = OL_NONE;  // the lane's ray, until its hit is written
   uint32_t nv = 0, nt = 0, ni = 0;
   while (true) {
-    const uint64_t idle = __ballot(!busy);
-    const uint32_t n_idle = (uint32_t)__popcll(idle);
-    if (n_idle >= kRefillMin2) {
+    uint64_t inner = lanes_where(item_is_inner(q.node)), leafy = lanes_where(item_is_leaf(q.node));
+    bool more = !(pool.exhausted && pool.n == 0);
+    if (more && (uint32_t)__popcll(inner | leafy) + kRefillMin2 <= 64u) {
+      if (q.node == OL_NONE && slot != OL_NONE) {
+        W.hit[slot] = make_float4(q.best.t, q.best.u, q.best.v, __uint_as_float(q.best.slot));
+        W.hit_inst[slot] = q.best_inst;
+        slot = OL_NONE;
+      }
       pool2_refill(pool, W, prefix, top, counts, cursor, c_begin, c_end);
-      const uint32_t take = min(n_idle, pool.n);
-      if (!busy) {
-        const uint32_t rank = lanes_below(idle);
-        if (rank < take) {
-          slot = pool.slot + rank;
-          job = pool.job;
-          const float4 o = qo[slot], d = qd[slot];
-          closest2_begin(q, mk3(o), mk3(d), o.w, d.w);
-          if (W.jobs[job].P.sc.node_count == 0) {
-            W.hit[slot] = make_float4(d.w, 0.0f, 0.0f, __uint_as_float(OL_NONE));
-          } else {
-            two_level_start(st);
-            busy = true;
-          }
+      const uint64_t idle = ~(inner | leafy);
+      const uint32_t take = min((uint32_t)__popcll(idle), pool.n);
+      const uint32_t rank = lanes_below(idle);
+      if (q.node == OL_NONE && rank < take) {
+        const uint32_t i = pool.slot + rank;
+        job = pool.job;
+        const DScene& sc = W.jobs[job].P.sc;
+        const float4 o = qo[i], d = qd[i];
+        if (sc.node_count == 0) {
+          W.hit[i] = make_float4(d.w, 0.0f, 0.0f, __uint_as_float(OL_NONE));
+        } else {
+          closest2_begin(sc, q, mk3(o), mk3(d), o.w, d.w);
+          slot = i;
+          two_level_start(st);
         }
       }
       pool.slot += take;
       pool.n -= take;
+      more = !(pool.exhausted && pool.n == 0);
+      inner = lanes_where(item_is_inner(q.node));
+      leafy = lanes_where(item_is_leaf(q.node));
     }
-    const bool at_leaf = busy && closest2_at_leaf(q);
-    const bool at_entry = busy && closest2_at_entry(q);
-    const uint64_t leafy = __ballot(at_leaf);
-    const uint64_t entries = __ballot(at_entry);
-    const uint64_t inner = __ballot(busy && !at_leaf && !at_entry);
-    const uint32_t n_busy = (uint32_t)__popcll(leafy | entries | inner);
-    if (n_busy == 0) {
-      if (pool.exhausted && pool.n == 0) break;
+    if ((inner | leafy) == 0) {
+      if (!more) break;
       continue;
     }
     // Leaf, entry or node step: a class runs when it holds a quarter of the
     // busy lanes or nothing else is left (leaves first, then entries).  A
     // quarter measured faster than a third or a fifth for both classes on
     // the instanced sphere field (the flat kernels keep a third).
-    if (leafy && ((entries | inner) == 0 || 4u * (uint32_t)__popcll(leafy) >= n_busy)) {
-      if (at_leaf) closest2_leaf<LSTACK>(q, st, nt);
-    } else if (entries && (inner == 0 || 4u * (uint32_t)__popcll(entries) >= n_busy)) {
-      if (at_entry) closest2_enter<LSTACK>(W.jobs[job].P.sc, q, st, ni);
-    } else if (inner) {
-      if (busy && !at_leaf && !at_entry) closest2_node<LSTACK>(W.jobs[job].P.sc, q, st, nv);
-    } else {
-      if (at_leaf) closest2_leaf<LSTACK>(q, st, nt);
+    uint64_t at_top = lanes_where(q.inst == OL_NONE);
+    uint32_t n_busy = (uint32_t)__popcll(inner | leafy);
+    while (inner != 0 && 4u * (uint32_t)__popcll(leafy & ~at_top) < n_busy &&
+           4u * (uint32_t)__popcll(leafy & at_top) < n_busy) {
+      nv += (uint32_t)__popcll(inner);
+      if (item_is_inner(q.node)) {
+        closest2_node<LSTACK>(q, st);
+        two_level_leave(W.jobs[job].P.sc, q, st);
+      }
+      inner = lanes_where(item_is_inner(q.node));
+      leafy = lanes_where(item_is_leaf(q.node));
+      at_top = lanes_where(q.inst == OL_NONE);
+      n_busy = (uint32_t)__popcll(inner | leafy);
+      if (more && n_busy + kRefillMin2 <= 64u) break;
     }
-    if (busy && q.node == OL_NONE) {
-      W.hit[slot] = make_float4(q.best.t, q.best.u, q.best.v, __uint_as_float(q.best.slot));
-      W.hit_inst[slot] = q.best_inst;
-      busy = false;
+    const uint64_t leaves = leafy & ~at_top, entries = leafy & at_top;
+    if (leaves != 0 && (4u * (uint32_t)__popcll(leaves) >= n_busy || (entries | inner) == 0)) {
+      if (item_is_leaf(q.node) && q.inst != OL_NONE) {
+        closest2_leaf<LSTACK>(q, st, nt);
+        two_level_leave(W.jobs[job].P.sc, q, st);
+      }
+    } else if (entries != 0 && (4u * (uint32_t)__popcll(entries) >= n_busy || inner == 0)) {
+      if (item_is_leaf(q.node) && q.inst == OL_NONE) closest2_enter<LSTACK>(W.jobs[job].P.sc, q, st, ni);
     }
   }
-  if (W.work && (nv | nt | ni)) {
-    atomicAdd(&W.work[0], (unsigned long long)nv);
-    atomicAdd(&W.work[1], (unsigned long long)nt);
-    atomicAdd(&W.work[4], (unsigned long long)ni);
+  if (slot != OL_NONE) {
+    W.hit[slot] = make_float4(q.best.t, q.best.u, q.best.v, __uint_as_float(q.best.slot));
+    W.hit_inst[slot] = q.best_inst;
+  }
+  if (W.work) {
+    if (nv && lane_id() == 0u) atomicAdd(&W.work[0], (unsigned long long)nv);
+    if (nt) atomicAdd(&W.work[1], (unsigned long long)nt);
+    if (ni) atomicAdd(&W.work[4], (unsigned long long)ni);
   }
 }
 
@@ -699,80 +735,93 @@ OL_DEV void shadow2_pass(const Wave& W, uint32_t in, TravStack<LSTACK>& st) {
   q.node = OL_NONE;
   q.inst = OL_NONE;
   q.occluded = false;
-  uint32_t job = 0, g = 0, e = 0, e_end = 0, mode = 0;
+  uint32_t job = 0, g = OL_NONE, e = 0, e_end = 0, mode = 0;  // the lane's group until it is resolved
   f3 direct = mk3(0.0f, 0.0f, 0.0f), area_direct = direct, env_direct = direct;
-  bool busy = false;
   uint32_t nv = 0, nt = 0, ni = 0;
   while (true) {
-    const uint64_t idle = __ballot(!busy);
-    const uint32_t n_idle = (uint32_t)__popcll(idle);
-    if (n_idle >= kRefillMin2) {
+    uint64_t inner = lanes_where(item_is_inner(q.node)), leafy = lanes_where(item_is_leaf(q.node));
+    bool more = !(pool.exhausted && pool.n == 0);
+    uint64_t ended = lanes_where(q.node == OL_NONE && g != OL_NONE);
+    if ((more || ended != 0) && (uint32_t)__popcll(inner | leafy) + kRefillMin2 <= 64u) {
+      if (q.node == OL_NONE && g != OL_NONE) {
+        if (!q.occluded) shadow_add(mode, W.ec[e], direct, area_direct, env_direct);
+        ++e;
+        if (e < e_end) {
+          const float4 o = W.eo[e], d = W.ed[e];
+          any2_begin(W.jobs[job].P.sc, q, mk3(o), mk3(d), o.w, d.w);
+          two_level_start(st);
+        } else {
+          shadow_resolve(W, g, direct, area_direct, env_direct);
+          g = OL_NONE;
+        }
+      }
       pool2_refill(pool, W, prefix, top, counts, cursor, c_begin, c_end);
-      const uint32_t take = min(n_idle, pool.n);
-      if (!busy) {
-        const uint32_t rank = lanes_below(idle);
-        if (rank < take) {
-          g = pool.slot + rank;
-          job = pool.job;
-          const uint4 gI = W.gI[g];
-          e = gI.y;
-          e_end = gI.y + gI.z;
-          mode = gI.w >> 16;
-          direct = mk3(0.0f, 0.0f, 0.0f);
-          area_direct = direct;
-          env_direct = direct;
-          if (W.jobs[job].P.sc.node_count == 0) {
-            for (; e < e_end; ++e) shadow_add(mode, W.ec[e], direct, area_direct, env_direct);
-            shadow_resolve(W, g, direct, area_direct, env_direct);
-          } else if (e < e_end) {
-            const float4 o = W.eo[e], d = W.ed[e];
-            any2_begin(q, mk3(o), mk3(d), o.w, d.w);
-            two_level_start(st);
-            busy = true;
-          } else {
-            shadow_resolve(W, g, direct, area_direct, env_direct);
-          }
+      const uint64_t idle = lanes_where(q.node == OL_NONE);
+      const uint32_t take = min((uint32_t)__popcll(idle), pool.n);
+      const uint32_t rank = lanes_below(idle);
+      if (q.node == OL_NONE && rank < take) {
+        g = pool.slot + rank;
+        job = pool.job;
+        const DScene& sc = W.jobs[job].P.sc;
+        const uint4 gI = W.gI[g];
+        e = gI.y;
+        e_end = gI.y + gI.z;
+        mode = gI.w >> 16;
+        direct = mk3(0.0f, 0.0f, 0.0f);
+        area_direct = direct;
+        env_direct = direct;
+        if (sc.node_count != 0 && e < e_end) {
+          const float4 o = W.eo[e], d = W.ed[e];
+          any2_begin(sc, q, mk3(o), mk3(d), o.w, d.w);
+          two_level_start(st);
+        } else {
+          for (; e < e_end; ++e) shadow_add(mode, W.ec[e], direct, area_direct, env_direct);
+          shadow_resolve(W, g, direct, area_direct, env_direct);
+          g = OL_NONE;
         }
       }
       pool.slot += take;
       pool.n -= take;
+      more = !(pool.exhausted && pool.n == 0);
+      inner = lanes_where(item_is_inner(q.node));
+      leafy = lanes_where(item_is_leaf(q.node));
+      ended = 0;
     }
-    const bool at_leaf = busy && any2_at_leaf(q);
-    const bool at_entry = busy && any2_at_entry(q);
-    const uint64_t leafy = __ballot(at_leaf);
-    const uint64_t entries = __ballot(at_entry);
-    const uint64_t inner = __ballot(busy && !at_leaf && !at_entry);
-    const uint32_t n_busy = (uint32_t)__popcll(leafy | entries | inner);
-    if (n_busy == 0) {
-      if (pool.exhausted && pool.n == 0) break;
+    if ((inner | leafy) == 0) {
+      if (!more && ended == 0) break;
       continue;
     }
-    if (leafy && ((entries | inner) == 0 || 4u * (uint32_t)__popcll(leafy) >= n_busy)) {
-      if (at_leaf) any2_leaf<LSTACK>(q, st, nt);
-    } else if (entries && (inner == 0 || 4u * (uint32_t)__popcll(entries) >= n_busy)) {
-      if (at_entry) any2_enter<LSTACK>(W.jobs[job].P.sc, q, st, ni);
-    } else if (inner) {
-      if (busy && !at_leaf && !at_entry) any2_node<LSTACK>(W.jobs[job].P.sc, q, st, nv);
-    } else {
-      if (at_leaf) any2_leaf<LSTACK>(q, st, nt);
-    }
-    if (busy && q.node == OL_NONE) {
-      if (!q.occluded) shadow_add(mode, W.ec[e], direct, area_direct, env_direct);
-      ++e;
-      if (e < e_end) {
-        const float4 o = W.eo[e], d = W.ed[e];
-        any2_begin(q, mk3(o), mk3(d), o.w, d.w);
-        two_level_start(st);
-      } else {
-        shadow_resolve(W, g, direct, area_direct, env_direct);
-        busy = false;
+    uint64_t at_top = lanes_where(q.inst == OL_NONE);
+    uint32_t n_busy = (uint32_t)__popcll(inner | leafy);
+    while (inner != 0 && 4u * (uint32_t)__popcll(leafy & ~at_top) < n_busy &&
+           4u * (uint32_t)__popcll(leafy & at_top) < n_busy) {
+      nv += (uint32_t)__popcll(inner);
+      if (item_is_inner(q.node)) {
+        any2_node<LSTACK>(q, st);
+        two_level_leave(W.jobs[job].P.sc, q, st);
       }
+      inner = lanes_where(item_is_inner(q.node));
+      leafy = lanes_where(item_is_leaf(q.node));
+      at_top = lanes_where(q.inst == OL_NONE);
+      const uint32_t left = (uint32_t)__popcll(inner | leafy);
+      const bool refill = left != n_busy && left + kRefillMin2 <= 64u;
+      n_busy = left;
+      if (refill) break;
+    }
+    const uint64_t leaves = leafy & ~at_top, entries = leafy & at_top;
+    if (leaves != 0 && (4u * (uint32_t)__popcll(leaves) >= n_busy || (entries | inner) == 0)) {
+      if (item_is_leaf(q.node) && q.inst != OL_NONE) {
+        any2_leaf<LSTACK>(q, st, nt);
+        two_level_leave(W.jobs[job].P.sc, q, st);
+      }
+    } else if (entries != 0 && (4u * (uint32_t)__popcll(entries) >= n_busy || inner == 0)) {
+      if (item_is_leaf(q.node) && q.inst == OL_NONE) any2_enter<LSTACK>(W.jobs[job].P.sc, q, st, ni);
     }
   }
-  if (W.work && (nv | nt | ni)) {
-    atomicAdd(&W.work[2], (unsigned long long)nv);
-    atomicAdd(&W.work[3], (unsigned long long)nt);
-    atomicAdd(&W.work[5], (unsigned long long)ni);
+  if (W.work) {
+    if (nv && lane_id() == 0u) atomicAdd(&W.work[2], (unsigned long long)nv);
+    if (nt) atomicAdd(&W.work[3], (unsigned long long)nt);
+    if (ni) atomicAdd(&W.work[5], (unsigned long long)ni);
   }
 }
 
@@ -837,12 +886,19 @@ __global__ void __launch_bounds__(BLOCK) k_trace_rays2(DScene sc, const float4* 
   for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) {
     const float4 o = o4[i], d = d4[i];
     Closest2 q;
-    closest2_begin(q, mk3(o), mk3(d), o.w, d.w);
+    closest2_begin(sc, q, mk3(o), mk3(d), o.w, d.w);
     two_level_start(st);
     if (sc.node_count == 0) q.node = OL_NONE;
     while (q.node != OL_NONE) {
-      if (closest2_at_leaf(q)) closest2_leaf<LSTACK>(q, st, nt);
-      else closest2_inner<LSTACK>(sc, q, st, nv, ni);
+      if (item_is_inner(q.node)) {
+        ++nv;
+        closest2_node<LSTACK>(q, st);
+      } else if (q.inst != OL_NONE) {
+        closest2_leaf<LSTACK>(q, st, nt);
+      } else {
+        closest2_enter<LSTACK>(sc, q, st, ni);
+      }
+      two_level_leave(sc, q, st);
     }
     hits[i] = make_float4(q.best.t, q.best.u, q.best.v, __uint_as_float(q.best.orig));
   }

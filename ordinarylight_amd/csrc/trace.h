@@ -255,8 +255,10 @@ OL_DEV void descend(TravStack<LSTACK>& st, const double p[4], uint32_t hits, uin
 // OL_NONE once the traversal has finished.  A wave chooses per step whether
 // its lanes at inner nodes or its lanes at leaves advance, so the triangle
 // tests of a leaf run with many lanes active instead of stalling the box
-// tests of the others.
-OL_DEV bool item_is_leaf(uint32_t item) { return child_is_leaf(item); }
+// tests of the others.  The item alone tells a lane's class, one signed
+// compare each: inner nodes are not negative, OL_NONE is -1.
+OL_DEV bool item_is_inner(uint32_t item) { return (int)item >= 0; }
+OL_DEV bool item_is_leaf(uint32_t item) { return (int)item < -1; }
 
 template <int LSTACK>
 OL_DEV void closest_next(ClosestRay& q, TravStack<LSTACK>& st) { q.node = st.empty() ? OL_NONE : st.pop(); }
@@ -264,10 +266,9 @@ OL_DEV void closest_next(ClosestRay& q, TravStack<LSTACK>& st) { q.node = st.emp
 // Inner step: continue with the nearest hit child (inner or leaf), the others
 // on the stack.
 template <int LSTACK>
-OL_DEV void closest_inner(const WideNode* __restrict__ nodes, ClosestRay& q, TravStack<LSTACK>& st, uint32_t& nv) {
+OL_DEV void closest_inner(const WideNode* __restrict__ nodes, ClosestRay& q, TravStack<LSTACK>& st) {
   uint4 w0, w1, w2, w3;
   load_node(nodes, q.node, w0, w1, w2, w3);
-  ++nv;
   double p[4];
   const uint32_t hits = node_children<true>(w0, w1, w2, w3, q.r, q.tmin, cull_distance(q.best.t), p);
   descend(st, p, hits, q.node);
@@ -316,10 +317,9 @@ template <int LSTACK>
 OL_DEV void any_next(AnyRay& q, TravStack<LSTACK>& st) { q.node = st.empty() ? OL_NONE : st.pop(); }
 
 template <int LSTACK>
-OL_DEV void any_inner(const WideNode* __restrict__ nodes, AnyRay& q, TravStack<LSTACK>& st, uint32_t& nv) {
+OL_DEV void any_inner(const WideNode* __restrict__ nodes, AnyRay& q, TravStack<LSTACK>& st) {
   uint4 w0, w1, w2, w3;
   load_node(nodes, q.node, w0, w1, w2, w3);
-  ++nv;
   double p[4];
   const uint32_t hits = node_children<false>(w0, w1, w2, w3, q.r, q.tmin, q.tcull, p);
   descend(st, p, hits, q.node);
@@ -353,8 +353,11 @@ OL_DEV TraceHit ol_trace_closest(const WideNode* __restrict__ nodes, const float
   if (node_count == 0) return q.best;
   st.sp = 0;
   while (q.node != OL_NONE) {
-    while (!child_is_leaf(q.node) && q.node != OL_NONE) closest_inner<LSTACK>(nodes, q, st, nv);
-    while (child_is_leaf(q.node)) closest_leaf<LSTACK>(tri, q, st, nt);
+    while (item_is_inner(q.node)) {
+      ++nv;
+      closest_inner<LSTACK>(nodes, q, st);
+    }
+    while (item_is_leaf(q.node)) closest_leaf<LSTACK>(tri, q, st, nt);
   }
   return q.best;
 }
@@ -461,11 +464,11 @@ struct Closest2 {
   uint32_t node;           // next item
   uint32_t inst;           // current instance, OL_NONE at the top level
   uint32_t offset;         // current instance's triangle offset
-  const WideNode* bnodes;  // current bottom-level BVH
-  const float4* btri;
+  const WideNode* nodes;   // current level's nodes
+  const float4* btri;      // current bottom level's triangles
 };
 
-OL_DEV void closest2_begin(Closest2& q, f3 o, f3 d, float tmin, float tmax) {
+OL_DEV void closest2_begin(const DScene& sc, Closest2& q, f3 o, f3 d, float tmin, float tmax) {
   q.w = ray_pre(o, d);
   q.r = q.w;
   q.tmin = tmin;
@@ -474,12 +477,12 @@ OL_DEV void closest2_begin(Closest2& q, f3 o, f3 d, float tmin, float tmax) {
   q.node = 0;
   q.inst = OL_NONE;
   q.offset = 0;
-  q.bnodes = nullptr;
+  q.nodes = sc.nodes;
   q.btri = nullptr;
 }
 
-// Leaf step: only bottom-level leaves (triangle tests in object space).
-OL_DEV bool closest2_at_leaf(const Closest2& q) { return q.inst != OL_NONE && child_is_leaf(q.node); }
+// Leaf steps are for bottom-level leaves only (triangle tests in object
+// space); a top-level leaf is an entry (below).
 
 template <int LSTACK>
 OL_DEV void closest2_next(Closest2& q, TravStack<LSTACK>& st) { q.node = st.empty() ? OL_NONE : st.pop(); }
@@ -488,8 +491,6 @@ OL_DEV void closest2_next(Closest2& q, TravStack<LSTACK>& st) { q.node = st.empt
 // enters it, in object space, unless its bounding sphere starts beyond the
 // best hit.  Kept apart from node steps, so that a wave runs the entry code
 // only for lanes that all enter (it is several times a node test's cost).
-OL_DEV bool closest2_at_entry(const Closest2& q) { return q.inst == OL_NONE && child_is_leaf(q.node); }
-
 template <int LSTACK>
 OL_DEV void closest2_enter(const DScene& sc, Closest2& q, TravStack<LSTACK>& st, uint32_t& ni) {
   const uint32_t k = leaf_first(q.node);  // the instance table is in top-level leaf order
@@ -507,36 +508,31 @@ OL_DEV void closest2_enter(const DScene& sc, Closest2& q, TravStack<LSTACK>& st,
   st.push(OL_SENTINEL);
   q.inst = k;
   q.offset = I.tri_offset;
-  q.bnodes = B.nodes;
+  q.nodes = B.nodes;
   q.btri = B.tri;
   q.r = ray_pre_fast(xform_point(I.w2o, q.w.o), xform_vector(I.w2o, q.w.d));
   q.node = I.root;
 }
 
-// Node step: leave an instance (sentinel) or test a node's boxes at the
-// current level.
+// Back to the top level where the sentinel has been taken off the stack,
+// and on to the next entry there.
+template <int LSTACK, class Ray>
+OL_DEV void two_level_leave(const DScene& sc, Ray& q, TravStack<LSTACK>& st) {
+  if (q.node != OL_SENTINEL) return;
+  q.inst = OL_NONE;
+  q.nodes = sc.nodes;
+  q.r = q.w;
+  q.node = st.empty() ? OL_NONE : st.pop();
+}
+
+// Node step: tests a node's boxes at the current level.
 template <int LSTACK>
-OL_DEV void closest2_node(const DScene& sc, Closest2& q, TravStack<LSTACK>& st, uint32_t& nv) {
-  if (q.node == OL_SENTINEL) {
-    q.inst = OL_NONE;
-    q.r = q.w;
-    closest2_next(q, st);
-    return;
-  }
-  const WideNode* nodes = q.inst == OL_NONE ? sc.nodes : q.bnodes;
+OL_DEV void closest2_node(Closest2& q, TravStack<LSTACK>& st) {
   uint4 w0, w1, w2, w3;
-  load_node(nodes, q.node, w0, w1, w2, w3);
-  ++nv;
+  load_node(q.nodes, q.node, w0, w1, w2, w3);
   double p[4];
   const uint32_t hits = node_children<true>(w0, w1, w2, w3, q.r, q.tmin, cull_distance(q.best.t), p);
   descend(st, p, hits, q.node);
-}
-
-// Entry or node step, whichever the lane is at.
-template <int LSTACK>
-OL_DEV void closest2_inner(const DScene& sc, Closest2& q, TravStack<LSTACK>& st, uint32_t& nv, uint32_t& ni) {
-  if (closest2_at_entry(q)) closest2_enter<LSTACK>(sc, q, st, ni);
-  else closest2_node<LSTACK>(sc, q, st, nv);
 }
 
 template <int LSTACK>
@@ -563,12 +559,12 @@ struct Any2 {
   RayPre w, r;
   float tmin, tmax, tcull;
   uint32_t node, inst;
-  const WideNode* bnodes;
+  const WideNode* nodes;
   const float4* btri;
   bool occluded;
 };
 
-OL_DEV void any2_begin(Any2& q, f3 o, f3 d, float tmin, float tmax) {
+OL_DEV void any2_begin(const DScene& sc, Any2& q, f3 o, f3 d, float tmin, float tmax) {
   q.w = ray_pre(o, d);
   q.r = q.w;
   q.tmin = tmin;
@@ -576,17 +572,13 @@ OL_DEV void any2_begin(Any2& q, f3 o, f3 d, float tmin, float tmax) {
   q.tcull = cull_distance(tmax);
   q.node = 0;
   q.inst = OL_NONE;
-  q.bnodes = nullptr;
+  q.nodes = sc.nodes;
   q.btri = nullptr;
   q.occluded = false;
 }
 
-OL_DEV bool any2_at_leaf(const Any2& q) { return q.inst != OL_NONE && child_is_leaf(q.node); }
-
 template <int LSTACK>
 OL_DEV void any2_next(Any2& q, TravStack<LSTACK>& st) { q.node = st.empty() ? OL_NONE : st.pop(); }
-
-OL_DEV bool any2_at_entry(const Any2& q) { return q.inst == OL_NONE && child_is_leaf(q.node); }
 
 template <int LSTACK>
 OL_DEV void any2_enter(const DScene& sc, Any2& q, TravStack<LSTACK>& st, uint32_t& ni) {
@@ -604,33 +596,19 @@ OL_DEV void any2_enter(const DScene& sc, Any2& q, TravStack<LSTACK>& st, uint32_
   ++ni;
   st.push(OL_SENTINEL);
   q.inst = k;
-  q.bnodes = B.nodes;
+  q.nodes = B.nodes;
   q.btri = B.tri;
   q.r = ray_pre_fast(xform_point(I.w2o, q.w.o), xform_vector(I.w2o, q.w.d));
   q.node = I.root;
 }
 
 template <int LSTACK>
-OL_DEV void any2_node(const DScene& sc, Any2& q, TravStack<LSTACK>& st, uint32_t& nv) {
-  if (q.node == OL_SENTINEL) {
-    q.inst = OL_NONE;
-    q.r = q.w;
-    any2_next(q, st);
-    return;
-  }
-  const WideNode* nodes = q.inst == OL_NONE ? sc.nodes : q.bnodes;
+OL_DEV void any2_node(Any2& q, TravStack<LSTACK>& st) {
   uint4 w0, w1, w2, w3;
-  load_node(nodes, q.node, w0, w1, w2, w3);
-  ++nv;
+  load_node(q.nodes, q.node, w0, w1, w2, w3);
   double p[4];
   const uint32_t hits = node_children<false>(w0, w1, w2, w3, q.r, q.tmin, q.tcull, p);
   descend(st, p, hits, q.node);
-}
-
-template <int LSTACK>
-OL_DEV void any2_inner(const DScene& sc, Any2& q, TravStack<LSTACK>& st, uint32_t& nv, uint32_t& ni) {
-  if (any2_at_entry(q)) any2_enter<LSTACK>(sc, q, st, ni);
-  else any2_node<LSTACK>(sc, q, st, nv);
 }
 
 template <int LSTACK>
