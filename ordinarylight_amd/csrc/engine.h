@@ -159,7 +159,8 @@ class Engine {
     uint64_t seq = 0;
     bool traced = false;  // traversal ran (otherwise accumulation only)
     bool timed = false;
-    int buf = 0;          // staging, report and event set of the step
+    int buf = 0;          // staging and event set of the step
+    int report = 0;       // host report buffer (traced steps)
     std::vector<uint64_t> finals;  // jobs whose last chunk this step accumulates
   };
   // Builds and queues the next step; false when there is nothing to do.
@@ -192,6 +193,7 @@ class Engine {
   uint32_t parity_ = 0;           // input queue of the next step
   uint64_t steps_ = 0;
   uint64_t seq_ = 0;              // sequence number of the next step queued
+  uint64_t traced_ = 0;           // traced steps queued
   std::deque<InFlight> inflight_;
   std::atomic<uint32_t> inflight_count_{0};  // inflight_.size() for readers without step_mu_
   uint64_t overflow_checked_from_ = 0;       // first step whose stack-overflow flag is still unhandled

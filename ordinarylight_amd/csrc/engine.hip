@@ -126,7 +126,7 @@ Engine::Engine(olhip_ctx* ctx, const olhip_engine_config& cfg) : ctx_(ctx), cfg_
   list_dev_.reserve(sizeof(StepList));
   ensure_buffers();
   launch_ = make_launch();
-  wave_clear(wave_, ctx_->stream);
+  wave_clear(wave_, 0u, ctx_->stream);
   OL_HIP_CHECK(hipStreamSynchronize(ctx_->stream));
   totals_.path_slots = slots_;
   totals_.entry_slots = eslots_;
@@ -488,7 +488,7 @@ void Engine::launch_step(uint32_t key, bool timed, int buf) {
       OL_HIP_CHECK(hipEventRecord(ev[2], s));
     }
   } else if (!timed) {
-    wave_trace(launch_, wave_, in, kinds, s);
+    wave_trace(launch_, wave_, in, kinds, gen, s);
     wave_shade(launch_, wave_, in, kinds, gen, s);
   } else {
     // Read when the step is retired (no synchronisation inside the step).
@@ -496,12 +496,12 @@ void Engine::launch_step(uint32_t key, bool timed, int buf) {
     for (int k = 0; k < 3; ++k)
       if (!ev[k]) OL_HIP_CHECK(hipEventCreate(&ev[k]));
     OL_HIP_CHECK(hipEventRecord(ev[0], s));
-    wave_trace(launch_, wave_, in, kinds, s);
+    wave_trace(launch_, wave_, in, kinds, gen, s);
     OL_HIP_CHECK(hipEventRecord(ev[1], s));
     wave_shade(launch_, wave_, in, kinds, gen, s);
     OL_HIP_CHECK(hipEventRecord(ev[2], s));
   }
-  wave_epilogue(wave_, in, s);
+  wave_epilogue(wave_, in, report_host_[0], report_host_[1], s);
 }
 
 void Engine::clear_graphs() {
@@ -704,10 +704,14 @@ bool Engine::launch_next() {
     OL_HIP_CHECK(hipGraphLaunch(graph_for(key), s));
   }
   OL_HIP_CHECK(hipGetLastError());
-  OL_HIP_CHECK(hipMemcpyAsync(report_host_[b], ctr_.as<uint32_t>() + C_OVERFLOW, 4ull * (C_WORDS - C_OVERFLOW),
-                              hipMemcpyDeviceToHost, s));
   OL_HIP_CHECK(hipEventRecord(done_[b], s));
-  if (traced) parity_ ^= 1u;
+  // The epilogue has written the step's report to the host buffer of the
+  // traced step count's parity.
+  f.report = (int)(traced_ & 1u);
+  if (traced) {
+    parity_ ^= 1u;
+    ++traced_;
+  }
   ++seq_;
   inflight_.push_back(std::move(f));
   return true;
@@ -745,7 +749,7 @@ void Engine::retire_front() {
     }
     if (f.traced) {
       ++steps_;
-      const uint32_t* report = report_host_[f.buf];
+      const uint32_t* report = report_host_[f.report];
       const uint32_t* rep = report + (C_REPORT - C_OVERFLOW);
       // The overflow flags are sticky until reset; a reset queued after an
       // overflow follows the steps already in flight, whose reports still
@@ -800,7 +804,7 @@ void Engine::retire_front() {
     // group counts (which a job admitted later into the same slot would
     // otherwise read as its own) and both flags.
     OL_HIP_CHECK(hipStreamSynchronize(ctx_->stream));
-    wave_clear(wave_, ctx_->stream);
+    wave_clear(wave_, (uint32_t)traced_, ctx_->stream);
     OL_HIP_CHECK(hipGetLastError());
     OL_HIP_CHECK(hipStreamSynchronize(ctx_->stream));
   }

@@ -82,7 +82,12 @@ constexpr uint32_t C_WS = C_W + kWorkStripes * kCursorStride;   // shadow cursor
 constexpr uint32_t C_W2 = C_WS + kWorkStripes * kCursorStride;  // closest-hit cursors (two-level)
 constexpr uint32_t C_WS2 = C_W2 + kWorkStripes * kCursorStride; // shadow cursors (two-level)
 constexpr uint32_t C_OVERFLOW = C_WS2 + kWorkStripes * kCursorStride, C_STACK = C_OVERFLOW + 1;
-constexpr uint32_t C_REPORT = C_OVERFLOW + 8;    // kMaxJobs x 4: rays traced, shadow rays, live paths, shaded hits
+// Steps traced since the counters were cleared (its parity picks the host
+// report buffer).
+constexpr uint32_t C_STEPS = C_OVERFLOW + 2;
+// Report layout (host buffers, from C_OVERFLOW on): the two overflow words,
+// then kMaxJobs x 4: rays traced, shadow rays, live paths, shaded hits.
+constexpr uint32_t C_REPORT = C_OVERFLOW + 8;
 constexpr uint32_t C_WORDS = C_REPORT + 4 * kMaxJobs;
 OL_HD constexpr uint32_t c_queue(uint32_t q) { return q ? C_Q1 : C_Q0; }
 OL_HD constexpr uint32_t c_groups(uint32_t p) { return p ? C_G1 : C_G0; }
@@ -218,15 +223,18 @@ void wave_accumulate(const Wave& w, int cu_count, hipStream_t st);
 // rays = false: queue counts and medium stacks only (the hybrid primary
 // kernel computes the camera rays itself).
 void wave_generate(const Wave& w, uint32_t in, int cu_count, hipStream_t st, bool rays = true);
-void wave_trace(const GiLaunch& l, const Wave& w, uint32_t in, uint32_t kinds, hipStream_t st);
+// `plan`: the step's input is not planned yet (it generates); otherwise the
+// previous step's epilogue has planned it.
+void wave_trace(const GiLaunch& l, const Wave& w, uint32_t in, uint32_t kinds, bool plan, hipStream_t st);
 // `gen`: the step generates (its step list holds the fresh slots).
 void wave_shade(const GiLaunch& l, const Wave& w, uint32_t in, uint32_t kinds, bool gen, hipStream_t st);
 // Hybrid primary step: plans the input queue and traces and shades it in one
 // kernel (every ray a fresh camera ray of a flat, untextured scene without
 // ReSTIR).
 void wave_primary(const GiLaunch& l, const Wave& w, uint32_t in, uint32_t kinds, hipStream_t st);
-void wave_epilogue(const Wave& w, uint32_t in, hipStream_t st);
-void wave_clear(const Wave& w, hipStream_t st);
+// Reports into host0 or host1 (pinned, by the parity of the steps traced).
+void wave_epilogue(const Wave& w, uint32_t in, uint32_t* host0, uint32_t* host1, hipStream_t st);
+void wave_clear(const Wave& w, uint32_t steps, hipStream_t st);
 
 // Closest hit of caller-supplied rays (primary-hit products, debugging).
 // Primary rays of a pixel tile (row-major) for the camera, size and frame in P.

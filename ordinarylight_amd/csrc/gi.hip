@@ -41,25 +41,28 @@ constexpr uint32_t kRefillMin = 16;
 constexpr uint32_t kRefillMin2 = 8;
 
 // ---- chunk plan ----------------------------------------------------------------------
-// Up to four plans in one launch, one block each: block b computes the
-// exclusive prefix of ceil(count / kChunk) over the runs of counter block
-// counts[b] whose jobs' scenes are flat (kind 0) or two-level (kind 1), into
-// out[b] (out[b][kRuns] = total), and the plan's bucket index (P_SHIFT ..
-// P_INDEX).  Offsets are counter-block words.
-struct PlanSet {
-  uint32_t counts[4], out[4], kind[4];
+// One plan, by a block of 1024 threads: the exclusive prefix of
+// ceil(count / kChunk) over the runs of a counter block whose jobs' scenes
+// are flat (kind 0) or two-level (kind 1), into out (out[kRuns] = total), and
+// the plan's bucket index (P_SHIFT .. P_INDEX).  kCapped: counts past a job's
+// append limit were reserved but not written, and do not count.
+// Each thread names one bucket's run by a bisection of the prefix in LDS:
+// filled run by run instead, a small job's single run left a thread writing
+// up to 1024 entries alone (30 us of a 250 us step of a 256 x 256 frame).
+struct PlanShared {
+  uint32_t prefix[kRuns], wave_tot[16], wave_last[16], shift;
 };
-
-__global__ void __launch_bounds__(1024) k_plan(uint32_t* __restrict__ ctr, const JobDev* __restrict__ jobs, PlanSet ps) {
+template <bool kCapped>
+OL_DEV void plan_runs(const uint32_t* __restrict__ counts, uint32_t* __restrict__ out, uint32_t kind,
+                      const JobDev* __restrict__ jobs, PlanShared& sh) {
   static_assert(kRuns == 2 * 1024 && kJobStripes % 2 == 0, "two runs of one job per thread");
-  __shared__ uint32_t wave_tot[16], wave_last[16], shift_s;
+  static_assert(kPlanBuckets == 1024, "one bucket per thread");
   const uint32_t t = threadIdx.x;
-  const uint32_t* __restrict__ counts = ctr + ps.counts[blockIdx.x];
-  uint32_t* __restrict__ out = ctr + ps.out[blockIdx.x];
-  const uint32_t kind = ps.kind[blockIdx.x];
-  const bool mine = (jobs[(2 * t) / kJobStripes].P.sc.instanced != 0u) == (kind != 0u);
-  const uint32_t a = mine ? (counts[run_word(2 * t)] + kChunk - 1u) / kChunk : 0u;
-  const uint32_t b = mine ? (counts[run_word(2 * t + 1)] + kChunk - 1u) / kChunk : 0u;
+  const JobDev& J = jobs[(2 * t) / kJobStripes];
+  const bool mine = (J.P.sc.instanced != 0u) == (kind != 0u);
+  const uint32_t cap = kCapped ? J.append : OL_NONE;
+  const uint32_t na = min(counts[run_word(2 * t)], cap), nb = min(counts[run_word(2 * t + 1)], cap);
+  const uint32_t a = mine ? (na + kChunk - 1u) / kChunk : 0u, b = mine ? (nb + kChunk - 1u) / kChunk : 0u;
   const uint32_t sum = a + b;
   uint32_t incl = sum;
   for (int off = 1; off < 64; off <<= 1) {
@@ -70,38 +73,58 @@ __global__ void __launch_bounds__(1024) k_plan(uint32_t* __restrict__ ctr, const
   uint32_t last = b ? 2u * t + 1u : (a ? 2u * t : 0u);
   for (int off = 32; off; off >>= 1) last = max(last, (uint32_t)__shfl_xor((int)last, off, 64));
   const uint32_t wave = t / 64u;
-  if (lane_id() == 63u) wave_tot[wave] = incl;
-  if (lane_id() == 0u) wave_last[wave] = last;
+  if (lane_id() == 63u) sh.wave_tot[wave] = incl;
+  if (lane_id() == 0u) sh.wave_last[wave] = last;
   __syncthreads();
-  uint32_t base = 0, total = 0;
+  uint32_t base = 0, total = 0, top = 0;
   for (uint32_t w = 0; w < 16u; ++w) {
-    if (w < wave) base += wave_tot[w];
-    total += wave_tot[w];
+    if (w < wave) base += sh.wave_tot[w];
+    total += sh.wave_tot[w];
+    top = max(top, sh.wave_last[w]);
   }
   const uint32_t excl = base + incl - sum;
+  sh.prefix[2 * t] = excl;
+  sh.prefix[2 * t + 1] = excl + a;
   out[2 * t] = excl;
   out[2 * t + 1] = excl + a;
+  // Buckets of 2^shift chunks, at most kPlanBuckets of them.
+  uint32_t shift = 0;
+  while (((total + (1u << shift) - 1u) >> shift) > kPlanBuckets) ++shift;
+  const uint32_t buckets = (total + (1u << shift) - 1u) >> shift;
   if (t == 0) {
-    uint32_t shift = 0;
-    while (((total + (1u << shift) - 1u) >> shift) > kPlanBuckets) ++shift;
-    uint32_t top = 0;
-    for (uint32_t w = 0; w < 16u; ++w) top = max(top, wave_last[w]);
     out[kRuns] = total;
     out[P_SHIFT] = shift;
-    out[P_BUCKETS] = (total + (1u << shift) - 1u) >> shift;
+    out[P_BUCKETS] = buckets;
     out[P_LAST] = top;
-    shift_s = shift;
   }
   __syncthreads();
-  // Bucket k starts at chunk k << shift; the run whose chunks hold that
-  // start names it (runs without chunks name none).
-  const uint32_t shift = shift_s;
-  const uint32_t firsts[2] = {excl, excl + a}, ns[2] = {a, b};
-  for (int h = 0; h < 2; ++h) {
-    if (ns[h] == 0u) continue;
-    const uint32_t p = firsts[h];
-    for (uint32_t k = (p + (1u << shift) - 1u) >> shift; k <= (p + ns[h] - 1u) >> shift; ++k) out[P_INDEX + k] = 2u * t + (uint32_t)h;
+  // Bucket t starts at chunk t << shift; the last run starting no later
+  // holds that chunk (runs without chunks start where the next one does).
+  if (t < buckets) {
+    const uint32_t chunk = t << shift;
+    uint32_t lo = 0, hi = top;
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi + 1u) >> 1;
+      if (sh.prefix[mid] <= chunk) lo = mid;
+      else hi = mid - 1u;
+    }
+    out[P_INDEX + t] = lo;
   }
+}
+
+// The four plans of a step: the input ray queue and the previous step's
+// shadow groups, each for flat and for two-level scenes (block k).
+template <bool kCapped>
+OL_DEV void plan_step(uint32_t* ctr, uint32_t in, uint32_t k, const JobDev* jobs, PlanShared& sh) {
+  const uint32_t out = k == 0u ? C_RP : (k == 1u ? C_GP : (k == 2u ? C_RP2 : C_GP2));
+  plan_runs<kCapped>(ctr + ((k & 1u) ? c_groups(in ^ 1u) : c_queue(in)), ctr + out, k >> 1, jobs, sh);
+}
+
+// Steps that generate plan after it; the others were planned by the
+// previous step's epilogue.
+__global__ void __launch_bounds__(1024) k_plan(uint32_t* ctr, uint32_t in, const JobDev* __restrict__ jobs) {
+  __shared__ PlanShared sh;
+  plan_step<false>(ctr, in, blockIdx.x, jobs, sh);
 }
 
 // A plan's bucket parameters, read once per kernel.
@@ -678,14 +701,14 @@ OL_DEV void closest2_pass(const Wave& W, uint32_t in, TravStack<LSTACK>& st) {
       if (!more) break;
       continue;
     }
-    // Leaf, entry or node step: a class runs when it holds a quarter of the
-    // busy lanes or nothing else is left (leaves first, then entries).  A
-    // quarter measured faster than a third or a fifth for both classes on
-    // the instanced sphere field (the flat kernels keep a third).
+    // Leaf, entry or node step: a class runs when it holds a third of the
+    // busy lanes or nothing else is left (leaves first, then entries).
+    // Instanced sphere field, traversal ms per frame: a third 48.5, a quarter
+    // 49.4, a fifth 51.5.
     uint64_t at_top = lanes_where(q.inst == OL_NONE);
     uint32_t n_busy = (uint32_t)__popcll(inner | leafy);
-    while (inner != 0 && 4u * (uint32_t)__popcll(leafy & ~at_top) < n_busy &&
-           4u * (uint32_t)__popcll(leafy & at_top) < n_busy) {
+    while (inner != 0 && 3u * (uint32_t)__popcll(leafy & ~at_top) < n_busy &&
+           3u * (uint32_t)__popcll(leafy & at_top) < n_busy) {
       nv += (uint32_t)__popcll(inner);
       if (item_is_inner(q.node)) {
         closest2_node<LSTACK>(q, st);
@@ -698,12 +721,12 @@ OL_DEV void closest2_pass(const Wave& W, uint32_t in, TravStack<LSTACK>& st) {
       if (more && n_busy + kRefillMin2 <= 64u) break;
     }
     const uint64_t leaves = leafy & ~at_top, entries = leafy & at_top;
-    if (leaves != 0 && (4u * (uint32_t)__popcll(leaves) >= n_busy || (entries | inner) == 0)) {
+    if (leaves != 0 && (3u * (uint32_t)__popcll(leaves) >= n_busy || (entries | inner) == 0)) {
       if (item_is_leaf(q.node) && q.inst != OL_NONE) {
         closest2_leaf<LSTACK>(q, st, nt);
         two_level_leave(W.jobs[job].P.sc, q, st);
       }
-    } else if (entries != 0 && (4u * (uint32_t)__popcll(entries) >= n_busy || inner == 0)) {
+    } else if (entries != 0 && (3u * (uint32_t)__popcll(entries) >= n_busy || inner == 0)) {
       if (item_is_leaf(q.node) && q.inst == OL_NONE) closest2_enter<LSTACK>(W.jobs[job].P.sc, q, st, ni);
     }
   }
@@ -793,8 +816,8 @@ OL_DEV void shadow2_pass(const Wave& W, uint32_t in, TravStack<LSTACK>& st) {
     }
     uint64_t at_top = lanes_where(q.inst == OL_NONE);
     uint32_t n_busy = (uint32_t)__popcll(inner | leafy);
-    while (inner != 0 && 4u * (uint32_t)__popcll(leafy & ~at_top) < n_busy &&
-           4u * (uint32_t)__popcll(leafy & at_top) < n_busy) {
+    while (inner != 0 && 3u * (uint32_t)__popcll(leafy & ~at_top) < n_busy &&
+           3u * (uint32_t)__popcll(leafy & at_top) < n_busy) {
       nv += (uint32_t)__popcll(inner);
       if (item_is_inner(q.node)) {
         any2_node<LSTACK>(q, st);
@@ -809,12 +832,12 @@ OL_DEV void shadow2_pass(const Wave& W, uint32_t in, TravStack<LSTACK>& st) {
       if (refill) break;
     }
     const uint64_t leaves = leafy & ~at_top, entries = leafy & at_top;
-    if (leaves != 0 && (4u * (uint32_t)__popcll(leaves) >= n_busy || (entries | inner) == 0)) {
+    if (leaves != 0 && (3u * (uint32_t)__popcll(leaves) >= n_busy || (entries | inner) == 0)) {
       if (item_is_leaf(q.node) && q.inst != OL_NONE) {
         any2_leaf<LSTACK>(q, st, nt);
         two_level_leave(W.jobs[job].P.sc, q, st);
       }
-    } else if (entries != 0 && (4u * (uint32_t)__popcll(entries) >= n_busy || inner == 0)) {
+    } else if (entries != 0 && (3u * (uint32_t)__popcll(entries) >= n_busy || inner == 0)) {
       if (item_is_leaf(q.node) && q.inst == OL_NONE) any2_enter<LSTACK>(W.jobs[job].P.sc, q, st, ni);
     }
   }
@@ -1728,23 +1751,34 @@ k_primary(Wave W, uint32_t in, uint32_t* spill, uint32_t spill_cap) {
 }
 
 // ---- step epilogue -----------------------------------------------------------------------------
-// Per-job report: rays traced from the input queue, shadow rays traced (the
-// previous step's entries), work left (paths in the output queue plus the
-// shadow groups this step's shading emitted, which the next step traces)
-// and shaded hits (those groups); then a reset of every consumed counter,
-// so the input queue and the traced groups can serve the next step's output.
-__global__ void __launch_bounds__(1024) k_epilogue(Wave W, uint32_t in) {
-  __shared__ uint32_t rep[4 * kMaxJobs];
+// Block 4: per-job report (rays traced from the input queue, shadow rays
+// traced (the previous step's entries), work left (paths in the output queue
+// plus the shadow groups this step's shading emitted, which the next step
+// traces) and shaded hits (those groups)), then a reset of every consumed
+// counter, so the input queue and the traced groups can serve the next
+// step's output.  Blocks 0..3: the next step's plans, from counters that
+// block 4 reads and at most lowers to the limit they apply themselves.  One launch does what a plan and an epilogue launch
+// did, and the report goes straight into one of two host buffers in turn
+// (a copy after the step and the gaps round it had cost 12 us a step).
+__global__ void __launch_bounds__(1024) k_epilogue(Wave W, uint32_t in, uint32_t* host0, uint32_t* host1) {
+  __shared__ union {
+    PlanShared plan;
+    uint32_t rep[4 * kMaxJobs];
+  } sh;
   const uint32_t t = threadIdx.x;
-  if (t < 4 * kMaxJobs) rep[t] = 0u;
+  if (blockIdx.x < 4u) {
+    plan_step<true>(W.ctr, in ^ 1u, blockIdx.x, W.jobs, sh.plan);
+    return;
+  }
+  if (t < 4 * kMaxJobs) sh.rep[t] = 0u;
   __syncthreads();
   for (uint32_t r = t; r < kRuns; r += blockDim.x) {
     const uint32_t job = r / kJobStripes;
     const uint32_t a = W.ctr[c_queue(in) + run_word(r)], e = W.ctr[c_entries(in ^ 1u) + run_word(r)];
-    uint32_t l = W.ctr[c_queue(in ^ 1u) + run_word(r)], g = W.ctr[c_groups(in) + run_word(r)];
     // A reservation past the segment's capacity was counted but not written
     // (shade flagged the overflow): the next step enumerates written entries only.
     const uint32_t cap = W.jobs[job].append;
+    uint32_t l = W.ctr[c_queue(in ^ 1u) + run_word(r)], g = W.ctr[c_groups(in) + run_word(r)];
     if (l > cap) {
       l = cap;
       W.ctr[c_queue(in ^ 1u) + run_word(r)] = cap;
@@ -1753,30 +1787,30 @@ __global__ void __launch_bounds__(1024) k_epilogue(Wave W, uint32_t in) {
       g = cap;
       W.ctr[c_groups(in) + run_word(r)] = cap;
     }
-    if (a) atomicAdd(&rep[4 * job + 0], a);
-    if (e) atomicAdd(&rep[4 * job + 1], e);
-    if (l + g) atomicAdd(&rep[4 * job + 2], l + g);
-    if (g) atomicAdd(&rep[4 * job + 3], g);
+    if (a) atomicAdd(&sh.rep[4 * job + 0], a);
+    if (e) atomicAdd(&sh.rep[4 * job + 1], e);
+    if (l + g) atomicAdd(&sh.rep[4 * job + 2], l + g);
+    if (g) atomicAdd(&sh.rep[4 * job + 3], g);
     W.ctr[c_queue(in) + run_word(r)] = 0u;
     W.ctr[c_groups(in ^ 1u) + run_word(r)] = 0u;
     W.ctr[c_entries(in ^ 1u) + run_word(r)] = 0u;
   }
   if (t < 4 * kWorkStripes) W.ctr[C_W + t * kCursorStride] = 0u;
-  // Chunk totals of the four plans: a plan left out of the next step (no
-  // resident job of its kind) must read as empty.
-  if (t == 0) {
-    W.ctr[C_RP + kRuns] = 0u;
-    W.ctr[C_GP + kRuns] = 0u;
-    W.ctr[C_RP2 + kRuns] = 0u;
-    W.ctr[C_GP2 + kRuns] = 0u;
-  }
   __syncthreads();
-  if (t < 4 * kMaxJobs) W.ctr[C_REPORT + t] = rep[t];
+  uint32_t* host = (W.ctr[C_STEPS] & 1u) ? host1 : host0;
+  auto report = [&](uint32_t word, uint32_t v) {
+    __hip_atomic_store(&host[word], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  };
+  if (t < 4 * kMaxJobs) report(C_REPORT - C_OVERFLOW + t, sh.rep[t]);
+  if (t < 2u) report(t, W.ctr[C_OVERFLOW + t]);
+  __syncthreads();
+  if (t == 0u) ++W.ctr[C_STEPS];
 }
 
-// Zeroes the whole counter block (engine start).
-__global__ void __launch_bounds__(1024) k_clear(Wave W) {
-  for (uint32_t i = threadIdx.x; i < C_WORDS; i += blockDim.x) W.ctr[i] = 0u;
+// Zeroes the whole counter block (engine start, after an overflow); `steps`
+// steps have been traced.
+__global__ void __launch_bounds__(1024) k_clear(Wave W, uint32_t steps) {
+  for (uint32_t i = threadIdx.x; i < C_WORDS; i += blockDim.x) W.ctr[i] = i == C_STEPS ? steps : 0u;
   if (W.work && threadIdx.x < kWorkWords) W.work[threadIdx.x] = 0ull;
 }
 
@@ -1890,7 +1924,9 @@ int stack_depth_for(uint32_t bvh_depth) {
 
 uint64_t trace_spill_words(const GiLaunch& l) { OL_STACK_DISPATCH(spill_words_for, l); }
 
-void wave_clear(const Wave& w, hipStream_t st) { hipLaunchKernelGGL(k_clear, dim3(1), dim3(1024), 0, st, w); }
+void wave_clear(const Wave& w, uint32_t steps, hipStream_t st) {
+  hipLaunchKernelGGL(k_clear, dim3(1), dim3(1024), 0, st, w, steps);
+}
 
 void build_shade_records(BvhOutput& b, const uint4* vidx, const float4* normals, uint32_t count, bool material,
                          hipStream_t st, const float4* face_in, const float* metal_in) {
@@ -1911,40 +1947,14 @@ void wave_generate(const Wave& w, uint32_t in, int cu_count, hipStream_t st, boo
   hipLaunchKernelGGL(k_generate, dim3((unsigned)(cu_count * 8)), dim3(256), 0, st, w, in, rays ? 1u : 0u);
 }
 
-void wave_trace(const GiLaunch& l, const Wave& w, uint32_t in, uint32_t kinds, hipStream_t st) {
-  // One launch plans the input ray queue and the previous step's shadow
-  // groups for each scene kind present.
-  PlanSet ps{};
-  uint32_t n = 0;
-  auto add = [&](uint32_t counts, uint32_t out, uint32_t kind) {
-    ps.counts[n] = counts;
-    ps.out[n] = out;
-    ps.kind[n] = kind;
-    ++n;
-  };
-  if (kinds & STEP_FLAT) {
-    add(c_queue(in), C_RP, 0u);
-    add(c_groups(in ^ 1u), C_GP, 0u);
-  }
-  if (kinds & STEP_INSTANCED) {
-    add(c_queue(in), C_RP2, 1u);
-    add(c_groups(in ^ 1u), C_GP2, 1u);
-  }
-  if (n == 0) return;
-  hipLaunchKernelGGL(k_plan, dim3(n), dim3(1024), 0, st, w.ctr, w.jobs, ps);
+void wave_trace(const GiLaunch& l, const Wave& w, uint32_t in, uint32_t kinds, bool plan, hipStream_t st) {
+  if (plan) hipLaunchKernelGGL(k_plan, dim3(4), dim3(1024), 0, st, w.ctr, in, w.jobs);
   if (kinds & STEP_FLAT) [&] { OL_STACK_DISPATCH(launch_trace, l, w, in, st); }();
   if (kinds & STEP_INSTANCED) [&] { OL_STACK_DISPATCH(launch_trace2, l, w, in, st); }();
 }
 
 void wave_primary(const GiLaunch& l, const Wave& w, uint32_t in, uint32_t kinds, hipStream_t st) {
-  PlanSet ps{};
-  ps.counts[0] = c_queue(in);
-  ps.out[0] = C_RP;
-  ps.kind[0] = 0u;
-  ps.counts[1] = c_groups(in ^ 1u);
-  ps.out[1] = C_GP;
-  ps.kind[1] = 0u;
-  hipLaunchKernelGGL(k_plan, dim3(2), dim3(1024), 0, st, w.ctr, w.jobs, ps);
+  hipLaunchKernelGGL(k_plan, dim3(4), dim3(1024), 0, st, w.ctr, in, w.jobs);
   OL_STACK_DISPATCH(launch_primary, l, w, in, (kinds & STEP_TWO_PASS) != 0u, st);
 }
 
@@ -1966,8 +1976,8 @@ void wave_shade(const GiLaunch& l, const Wave& w, uint32_t in, uint32_t kinds, b
   }
 }
 
-void wave_epilogue(const Wave& w, uint32_t in, hipStream_t st) {
-  hipLaunchKernelGGL(k_epilogue, dim3(1), dim3(1024), 0, st, w, in);
+void wave_epilogue(const Wave& w, uint32_t in, uint32_t* host0, uint32_t* host1, hipStream_t st) {
+  hipLaunchKernelGGL(k_epilogue, dim3(5), dim3(1024), 0, st, w, in, host0, host1);
 }
 
 void camera_rays(const GiParams& P, uint32_t x0, uint32_t y0, uint32_t tw, uint32_t th, uint32_t sample, float4* o,
