@@ -907,7 +907,9 @@ int olhip_render_products(olhip_ctx* ctx, const olhip_scene* sc, const olhip_cam
       olhip_engine_config cfg{};
       cfg.path_slots = need;
       cfg.entry_factor = per_hit;
-      cfg.use_graph = 1;
+      // A lone job's step is three launches: launched directly they follow
+      // the previous step after 10 us, as a captured graph after 18.
+      cfg.use_graph = 0;
       cfg.fused_primary = (uint32_t)ctx->fused_primary;
       ctx->frame_engine = std::make_unique<Engine>(ctx, cfg);
       ctx->frame_engine_slots = need;

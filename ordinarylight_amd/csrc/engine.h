@@ -161,6 +161,7 @@ class Engine {
     bool timed = false;
     int buf = 0;          // staging and event set of the step
     int report = 0;       // host report buffer (traced steps)
+    hipEvent_t begin = nullptr, done = nullptr;  // the step's device time
     std::vector<uint64_t> finals;  // jobs whose last chunk this step accumulates
   };
   // Builds and queues the next step; false when there is nothing to do.
@@ -203,8 +204,8 @@ class Engine {
   bool tex_needed_ = false;
 
   // Device state.
-  DevBuf T_, L_, M_, stk_, rsamp_, tex_, cone_, qo_[2], qd_[2], qp_[2], hit_, hit_inst_, gT_, gI_, eo_, ed_, ec_, ctr_, work_, jobs_dev_,
-      list_dev_, spill_;
+  DevBuf T_, L_, M_, stk_, rsamp_, tex_, cone_, qo_[2], qd_[2], qp_[2], hit_, hit_inst_, gT_, gI_, eo_, ed_, ec_, ctr_, work_, stage_dev_,
+      spill_;
   uint64_t slots_ = 0, eslots_ = 0;
   Wave wave_{};
   GiLaunch launch_{};
@@ -216,11 +217,14 @@ class Engine {
   // pinned staging, one set per in-flight step.
   std::vector<JobDev> jobs_state_;
   bool jobs_dirty_ = true;
-  JobDev* jobs_host_[2] = {nullptr, nullptr};
-  StepList* list_host_[2] = {nullptr, nullptr};
+  StepStage* stage_host_[2] = {nullptr, nullptr};
   uint32_t* report_host_[2] = {nullptr, nullptr};
-  hipEvent_t done_[2] = {nullptr, nullptr};
-  hipEvent_t begin_[2] = {nullptr, nullptr};  // step start on the stream (device-time accounting)
+  // Ends of the last steps (two may be in flight, and each may serve the
+  // step behind it as its start), and the start of a step after an idle
+  // device (device-time accounting).
+  static constexpr uint64_t kEvents = 4;
+  hipEvent_t done_[kEvents] = {};
+  hipEvent_t begin_ = nullptr;
   hipEvent_t prof_ev_[2][3] = {{nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
   double t0_ms_ = 0;
   // Engine totals.

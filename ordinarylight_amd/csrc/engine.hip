@@ -112,18 +112,16 @@ Engine::Engine(olhip_ctx* ctx, const olhip_engine_config& cfg) : ctx_(ctx), cfg_
   entries_.reset(eslots_);
   jobs_state_.assign(kMaxJobs, JobDev{});
   for (int b = 0; b < 2; ++b) {
-    jobs_host_[b] = pinned<JobDev>(kMaxJobs);
-    list_host_[b] = pinned<StepList>(1);
+    stage_host_[b] = pinned<StepStage>(1);
     report_host_[b] = pinned<uint32_t>(C_WORDS - C_OVERFLOW);
-    OL_HIP_CHECK(hipEventCreate(&done_[b]));
-    OL_HIP_CHECK(hipEventCreate(&begin_[b]));
   }
+  OL_HIP_CHECK(hipEventCreate(&begin_));
+  for (hipEvent_t& e : done_) OL_HIP_CHECK(hipEventCreate(&e));
   t0_ms_ = 0;
   t0_ms_ = now_ms();
   ctr_.reserve(4ull * C_WORDS);
   work_.reserve(64);
-  jobs_dev_.reserve(sizeof(JobDev) * kMaxJobs);
-  list_dev_.reserve(sizeof(StepList));
+  stage_dev_.reserve(sizeof(StepStage));
   ensure_buffers();
   launch_ = make_launch();
   wave_clear(wave_, 0u, ctx_->stream);
@@ -139,13 +137,13 @@ Engine::~Engine() {
   // Jobs never taken leave their buffers to the context's pool.
   for (auto& kv : jobs_) keep_buffers(*kv.second);
   for (auto& kv : graphs_) (void)hipGraphExecDestroy(kv.second);
+  if (begin_) (void)hipEventDestroy(begin_);
+  for (hipEvent_t e : done_)
+    if (e) (void)hipEventDestroy(e);
   for (int b = 0; b < 2; ++b) {
-    if (done_[b]) (void)hipEventDestroy(done_[b]);
-    if (begin_[b]) (void)hipEventDestroy(begin_[b]);
     for (auto& x : prof_ev_[b])
       if (x) (void)hipEventDestroy(x);
-    if (jobs_host_[b]) (void)hipHostFree(jobs_host_[b]);
-    if (list_host_[b]) (void)hipHostFree(list_host_[b]);
+    if (stage_host_[b]) (void)hipHostFree(stage_host_[b]);
     if (report_host_[b]) (void)hipHostFree(report_host_[b]);
   }
 }
@@ -183,8 +181,8 @@ void Engine::ensure_buffers() {
     cone_.reserve(8 * slots_);
   }
   Wave w{};
-  w.jobs = jobs_dev_.as<JobDev>();
-  w.list = list_dev_.as<StepList>();
+  w.jobs = stage_dev_.as<StepStage>()->jobs;
+  w.list = &stage_dev_.as<StepStage>()->list;
   w.T = T_.as<float4>();
   w.L = L_.as<float4>();
   w.M = M_.as<uint4>();
@@ -578,7 +576,7 @@ uint32_t Engine::step() {
 // empty launches.
 bool Engine::launch_next() {
   const int b = (int)(seq_ & 1u);
-  StepList& Ls = *list_host_[b];
+  StepList& Ls = stage_host_[b]->list;
   bool traced = false, all_fresh = true;
   uint32_t kinds = 0;
   InFlight f;
@@ -675,15 +673,16 @@ bool Engine::launch_next() {
   }
   if (!traced && Ls.n_acc == 0) return false;
   hipStream_t s = ctx_->stream;
-  OL_HIP_CHECK(hipEventRecord(begin_[b], s));
-  if (jobs_dirty_) {
-    std::memcpy(jobs_host_[b], jobs_state_.data(), sizeof(JobDev) * kMaxJobs);
-    OL_HIP_CHECK(hipMemcpyAsync(jobs_dev_.ptr, jobs_host_[b], sizeof(JobDev) * kMaxJobs, hipMemcpyHostToDevice, s));
-    jobs_dirty_ = false;
-  }
-  // Only accumulation and generation read the step list.
-  if (Ls.n_acc || Ls.n_gen)
-    OL_HIP_CHECK(hipMemcpyAsync(list_dev_.ptr, list_host_[b], sizeof(StepList), hipMemcpyHostToDevice, s));
+  // A step queued behind another starts where that one ends; only a step
+  // after an idle device needs an event of its own for its start.
+  f.begin = inflight_.empty() ? begin_ : done_[(seq_ + kEvents - 1u) % kEvents];
+  if (inflight_.empty()) OL_HIP_CHECK(hipEventRecord(begin_, s));
+  // Only accumulation and generation read the step list, and the job table
+  // changes with an admission, which generates.
+  if (jobs_dirty_) std::memcpy(stage_host_[b]->jobs, jobs_state_.data(), sizeof(JobDev) * kMaxJobs);
+  if (jobs_dirty_ || Ls.n_acc || Ls.n_gen)
+    wave_stage(stage_host_[b], stage_dev_.as<StepStage>(), jobs_dirty_, s);
+  jobs_dirty_ = false;
   const uint32_t in = parity_;
   f.traced = traced;
   f.timed = traced && profiling_;
@@ -704,7 +703,8 @@ bool Engine::launch_next() {
     OL_HIP_CHECK(hipGraphLaunch(graph_for(key), s));
   }
   OL_HIP_CHECK(hipGetLastError());
-  OL_HIP_CHECK(hipEventRecord(done_[b], s));
+  f.done = done_[seq_ % kEvents];
+  OL_HIP_CHECK(hipEventRecord(f.done, s));
   // The epilogue has written the step's report to the host buffer of the
   // traced step count's parity.
   f.report = (int)(traced_ & 1u);
@@ -724,9 +724,9 @@ bool Engine::launch_next() {
 void Engine::retire_front() {
   InFlight f = std::move(inflight_.front());
   inflight_.pop_front();
-  OL_HIP_CHECK(hipEventSynchronize(done_[f.buf]));
+  OL_HIP_CHECK(hipEventSynchronize(f.done));
   float step_ms = 0.0f;
-  OL_HIP_CHECK(hipEventElapsedTime(&step_ms, begin_[f.buf], done_[f.buf]));
+  OL_HIP_CHECK(hipEventElapsedTime(&step_ms, f.begin, f.done));
   if (f.timed) {
     float a = 0, b = 0;
     OL_HIP_CHECK(hipEventElapsedTime(&a, prof_ev_[f.buf][0], prof_ev_[f.buf][1]));

@@ -149,6 +149,13 @@ struct StepList {
   AccItem acc[kMaxJobs];
 };
 
+// What a step needs from the host: the work lists, then the job table.  One
+// pinned copy per step in flight and one on the device.
+struct alignas(16) StepStage {
+  StepList list;
+  alignas(16) JobDev jobs[kMaxJobs];
+};
+
 // Device pointers of an engine (kernel argument).
 struct Wave {
   const JobDev* jobs;
@@ -219,6 +226,9 @@ constexpr uint32_t kStepKinds = 31u;
 // word 11).
 void build_shade_records(BvhOutput& b, const uint4* vidx, const float4* normals, uint32_t count, bool material,
                          hipStream_t st, const float4* face_in = nullptr, const float* metal_in = nullptr);
+// Brings the step lists, and the job table with `jobs`, from the pinned host
+// copy to the device copy.
+void wave_stage(const StepStage* host, StepStage* dev, bool jobs, hipStream_t st);
 void wave_accumulate(const Wave& w, int cu_count, hipStream_t st);
 // rays = false: queue counts and medium stacks only (the hybrid primary
 // kernel computes the camera rays itself).

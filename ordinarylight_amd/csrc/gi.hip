@@ -24,6 +24,7 @@
 // report after it.
 
 #include <algorithm>
+#include <cstddef>
 
 #include "gi.h"
 #include "shade.h"
@@ -174,6 +175,15 @@ OL_DEV uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); 
 OL_DEV uint32_t wave_sum(uint32_t v) {
   for (int off = 32; off; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
+}
+
+// ---- step staging ----------------------------------------------------------------------------
+// Copies a step's host data to the device as one launch on the step's
+// stream.  Two hipMemcpyAsync calls did it before, each a copy kernel of the
+// runtime's with 4 to 9 us of signals round it.
+__global__ void __launch_bounds__(256) k_stage(const uint4* __restrict__ host, uint4* __restrict__ dev, uint32_t n) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i < n) dev[i] = host[i];
 }
 
 // ---- accumulate + generate (host lists) ------------------------------------------------------
@@ -1937,6 +1947,13 @@ void build_shade_records(BvhOutput& b, const uint4* vidx, const float4* normals,
                      count, material ? 1u : 0u, b.shade.as<float4>(), face_in, metal_in,
                      face_in ? b.face.as<float4>() : nullptr);
   OL_HIP_CHECK(hipGetLastError());
+}
+
+void wave_stage(const StepStage* host, StepStage* dev, bool jobs, hipStream_t st) {
+  static_assert(offsetof(StepStage, jobs) % 16 == 0 && sizeof(StepStage) % 16 == 0, "copied in 16-byte words");
+  const uint32_t n = (uint32_t)((jobs ? sizeof(StepStage) : offsetof(StepStage, jobs)) / 16u);
+  hipLaunchKernelGGL(k_stage, dim3((n + 255u) / 256u), dim3(256), 0, st, reinterpret_cast<const uint4*>(host),
+                     reinterpret_cast<uint4*>(dev), n);
 }
 
 void wave_accumulate(const Wave& w, int cu_count, hipStream_t st) {
