@@ -261,27 +261,58 @@ __global__ void __launch_bounds__(kBlock) k_leaf_boxes(const uint32_t* __restric
   lmax[k] = make_float4(fmaxf(fmaxf(a.x, b.x), c.x), fmaxf(fmaxf(a.y, b.y), c.y), fmaxf(fmaxf(a.z, b.z), c.z), 0.0f);
 }
 
+// A box written by one thread and read by another one of the same kernel, on
+// any XCD: words that go through to the coherent level (agent-scope relaxed
+// stores and loads), so neither side flushes or invalidates a cache.
+__device__ __forceinline__ void put_box(float4* p, float x, float y, float z) {
+  uint64_t* w = reinterpret_cast<uint64_t*>(p);
+  const uint64_t xy = __float_as_uint(x) | ((uint64_t)__float_as_uint(y) << 32);
+  __hip_atomic_store(w, xy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(w + 1, (uint64_t)__float_as_uint(z), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ f3 get_box(const float4* p) {
+  uint64_t* w = reinterpret_cast<uint64_t*>(const_cast<float4*>(p));
+  const uint64_t xy = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint64_t z = __hip_atomic_load(w + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return mk3(__uint_as_float((uint32_t)xy), __uint_as_float((uint32_t)(xy >> 32)), __uint_as_float((uint32_t)z));
+}
+
+// One thread per leaf climbs while it is the second to arrive at a node, and
+// carries its subtree's box in registers; only the sibling's box is read.
+// Bound by the latency of the climb (one atomic and one box per level).
+//
+// A box is complete in the coherent level (the wait) before its subtree is
+// counted at the parent.  The count itself orders nothing: as an
+// acquire-release atomic it flushed and invalidated the XCD's cache at every
+// step, and the compiler left out the wait between that flush and the
+// atomic, so that a sibling's box was read before it had arrived in one of
+// some 200 builds of 62 500 triangles.
 __global__ void __launch_bounds__(kBlock) k_bottom_up(uint32_t n, const uint32_t* __restrict__ left,
                                                       const uint32_t* __restrict__ right,
                                                       const uint32_t* __restrict__ parent_int,
                                                       const uint32_t* __restrict__ parent_leaf,
                                                       const float4* __restrict__ lmin, const float4* __restrict__ lmax,
                                                       float4* bmin, float4* bmax, uint32_t* flags) {
-  uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+  const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
   if (k >= n) return;
-  uint32_t node = parent_leaf[k];
+  uint32_t node = parent_leaf[k], self = k | OL_LEAF_BIT;
+  f3 mn = mk3(lmin[k]), mx = mk3(lmax[k]);
   while (node != OL_NONE) {
-    // Release this subtree's box, acquire the sibling's (device scope).
-    uint32_t old = __hip_atomic_fetch_add(&flags[node], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-    if (old == 0) return;  // the sibling subtree finishes this node
-    float4 amn, amx, bmn, bmx;
-    ref_box(left[node], lmin, lmax, bmin, bmax, amn, amx);
-    ref_box(right[node], lmin, lmax, bmin, bmax, bmn, bmx);
-    float4 mn = make_float4(fminf(amn.x, bmn.x), fminf(amn.y, bmn.y), fminf(amn.z, bmn.z), 0.0f);
-    float4 mx = make_float4(fmaxf(amx.x, bmx.x), fmaxf(amx.y, bmx.y), fmaxf(amx.z, bmx.z), 0.0f);
-    bmin[node] = mn;
-    bmax[node] = mx;
-    node = parent_int[node];
+    const uint32_t l = left[node], r = right[node], up = parent_int[node];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this subtree's box has arrived
+    const uint32_t old = __hip_atomic_fetch_add(&flags[node], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::: "memory");
+    if (old == 0u) return;  // the sibling subtree finishes this node
+    const uint32_t other = l == self ? r : l, slot = other & ~OL_LEAF_BIT;
+    const bool leaf = (other & OL_LEAF_BIT) != 0u;
+    const f3 omn = leaf ? mk3(lmin[slot]) : get_box(bmin + slot);
+    const f3 omx = leaf ? mk3(lmax[slot]) : get_box(bmax + slot);
+    mn = mk3(fminf(mn.x, omn.x), fminf(mn.y, omn.y), fminf(mn.z, omn.z));
+    mx = mk3(fmaxf(mx.x, omx.x), fmaxf(mx.y, omx.y), fmaxf(mx.z, omx.z));
+    put_box(bmin + node, mn.x, mn.y, mn.z);
+    put_box(bmax + node, mx.x, mx.y, mx.z);
+    self = node;
+    node = up;
   }
 }
 
