@@ -274,6 +274,7 @@ int olhip_create(int device, olhip_ctx** out) {
     OL_HIP_CHECK(hipGetDeviceProperties(&prop, device));
     ctx->cu_count = prop.multiProcessorCount;
     ctx->trace_scratch = trace_scratch_address(device);
+    ctx->copier = std::make_unique<HostCopier>(device);
     *out = ctx.release();
   });
 }
@@ -285,6 +286,7 @@ int olhip_destroy(olhip_ctx* ctx) {
     ctx->frame_engine.reset();
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamDestroy(ctx->stream);
+    if (ctx->query_host) (void)hipHostFree(ctx->query_host);
     delete ctx;
   });
 }
@@ -937,7 +939,13 @@ int olhip_render_products(olhip_ctx* ctx, const olhip_scene* sc, const olhip_cam
     Event e_start, e_end;
     OL_HIP_CHECK(hipEventRecord(e_start.e, ctx->stream));
     const uint64_t id = eng.submit(d);
-    eng.run_until_idle();
+    Prefault outputs;
+    outputs.add(variance, sizeof(float) * np);
+    outputs.add(primitive, sizeof(uint32_t) * np);
+    outputs.add(normal, sizeof(float) * 3 * np);
+    outputs.add(depth, sizeof(float) * np);
+    outputs.add(out_rgba, sizeof(float4) * np);
+    eng.run_until_idle(&outputs);
     OL_HIP_CHECK(hipEventRecord(e_end.e, ctx->stream));
     OL_HIP_CHECK(hipEventSynchronize(e_end.e));
     olhip_job_stats js{};
@@ -952,7 +960,7 @@ int olhip_render_products(olhip_ctx* ctx, const olhip_scene* sc, const olhip_cam
     ctx->image_width = width;
     ctx->image_height = height;
     if (d.products) eng.products(id, depth, normal, primitive, variance);
-    if (out_rgba) OL_HIP_CHECK(hipMemcpy(out_rgba, ctx->image.ptr, sizeof(float4) * np, hipMemcpyDeviceToHost));
+    if (out_rgba) ctx->copier->download(out_rgba, ctx->image.ptr, sizeof(float4) * np);
     eng.take_result(id, nullptr, &js);
     if (stats_out) {
       olhip_stats& o = *stats_out;
@@ -1104,7 +1112,7 @@ int olhip_frame_download(olhip_ctx* ctx, float* out_rgba) {
     require(ctx->image_pixels > 0, "no frame has been rendered");
     OL_HIP_CHECK(hipSetDevice(ctx->device));
     OL_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-    OL_HIP_CHECK(hipMemcpy(out_rgba, ctx->image.ptr, sizeof(float4) * ctx->image_pixels, hipMemcpyDeviceToHost));
+    ctx->copier->download(out_rgba, ctx->image.ptr, sizeof(float4) * ctx->image_pixels);
   });
 }
 
@@ -1133,10 +1141,65 @@ int olhip_frame_output(olhip_ctx* ctx, uint32_t format, float exposure, uint32_t
     launch_output(format, ctx->image.as<float4>(), ctx->image_width, ctx->image_height, width, height, exposure, dst,
                   s);
     OL_HIP_CHECK(hipGetLastError());
-    if (!out_on_device) OL_HIP_CHECK(hipMemcpyAsync(out, staging.ptr, bytes, hipMemcpyDeviceToHost, s));
     OL_HIP_CHECK(hipStreamSynchronize(s));
+    if (!out_on_device) ctx->copier->download(out, staging.ptr, bytes);
   });
 }
+
+}  // extern "C"
+
+namespace {
+
+// Ray and hit buffers of one query, held under the context's lock.  Up to
+// kQueryDirect rays go through pinned memory that the kernel reads and writes
+// itself: no copy, no allocation (a pick had spent nine tenths of its 146 us
+// on four allocations and five copies).  Larger queries use device buffers
+// kept with the context while they stay under kQueryKeep bytes.
+struct QueryBuffers {
+  static constexpr uint32_t kQueryDirect = 4096;
+  static constexpr size_t kQueryKeep = size_t(256) << 20;
+  olhip_ctx* ctx;
+  uint32_t n;
+  std::lock_guard<std::mutex> lock;
+  bool direct;
+  float4 *o = nullptr, *d = nullptr, *h = nullptr;
+  uint32_t* overflow = nullptr;
+
+  QueryBuffers(olhip_ctx* c, uint32_t count) : ctx(c), n(count), lock(c->query_mu), direct(count <= kQueryDirect) {
+    if (!ctx->query_host) {
+      void* p = nullptr;
+      OL_HIP_CHECK(hipHostMalloc(&p, sizeof(float4) * 3 * kQueryDirect + 16, hipHostMallocDefault));
+      ctx->query_host = static_cast<float4*>(p);
+    }
+    overflow = reinterpret_cast<uint32_t*>(ctx->query_host + 3 * kQueryDirect);
+    if (direct) {
+      o = ctx->query_host;
+      d = o + kQueryDirect;
+      h = d + kQueryDirect;
+      return;
+    }
+    for (DevBuf* b : {&ctx->query_o, &ctx->query_d, &ctx->query_h}) b->reserve(sizeof(float4) * (size_t)n);
+    o = ctx->query_o.as<float4>();
+    d = ctx->query_d.as<float4>();
+    h = ctx->query_h.as<float4>();
+  }
+  ~QueryBuffers() {
+    if (ctx->query_o.bytes + ctx->query_d.bytes + ctx->query_h.bytes > kQueryKeep)
+      for (DevBuf* b : {&ctx->query_o, &ctx->query_d, &ctx->query_h}) b->release();
+  }
+  void put(float4* to, const float* from) {
+    if (direct) std::memcpy(to, from, sizeof(float4) * (size_t)n);
+    else OL_HIP_CHECK(hipMemcpyAsync(to, from, sizeof(float4) * (size_t)n, hipMemcpyHostToDevice, ctx->stream));
+  }
+  void get(float* to, const float4* from) {
+    if (direct) std::memcpy(to, from, sizeof(float4) * (size_t)n);
+    else ctx->copier->download(to, from, sizeof(float4) * (size_t)n);
+  }
+};
+
+}  // namespace
+
+extern "C" {
 
 int olhip_camera_rays(olhip_ctx* ctx, const olhip_camera* cam, uint32_t width, uint32_t height, uint32_t frame_index,
                       uint32_t sample, uint32_t x0, uint32_t y0, uint32_t tile_width, uint32_t tile_height,
@@ -1163,14 +1226,12 @@ int olhip_camera_rays(olhip_ctx* ctx, const olhip_camera* cam, uint32_t width, u
     P.height = height;
     P.frame = (uint32_t)((float)frame_index + 0.5f);
     const uint32_t n = tile_width * tile_height;
-    DevBuf o, d;
-    o.reserve(sizeof(float4) * n);
-    d.reserve(sizeof(float4) * n);
-    camera_rays(P, x0, y0, tile_width, tile_height, sample, o.as<float4>(), d.as<float4>(), s);
+    QueryBuffers q(ctx, n);
+    camera_rays(P, x0, y0, tile_width, tile_height, sample, q.o, q.d, s);
     OL_HIP_CHECK(hipGetLastError());
-    OL_HIP_CHECK(hipMemcpyAsync(origins, o.ptr, sizeof(float4) * n, hipMemcpyDeviceToHost, s));
-    OL_HIP_CHECK(hipMemcpyAsync(directions, d.ptr, sizeof(float4) * n, hipMemcpyDeviceToHost, s));
     OL_HIP_CHECK(hipStreamSynchronize(s));
+    q.get(origins, q.o);
+    q.get(directions, q.d);
   });
 }
 
@@ -1182,20 +1243,16 @@ int olhip_trace(olhip_ctx* ctx, const olhip_scene* sc, const float* origins, con
     if (n == 0) return;
     OL_HIP_CHECK(hipSetDevice(ctx->device));
     hipStream_t s = ctx->stream;
-    DevBuf o, d, h, ov;
-    upload(o, reinterpret_cast<const float4*>(origins), n, s);
-    upload(d, reinterpret_cast<const float4*>(directions), n, s);
-    h.reserve(sizeof(float4) * n);
-    ov.reserve(4);
-    OL_HIP_CHECK(hipMemsetAsync(ov.ptr, 0, 4, s));
+    QueryBuffers q(ctx, n);
+    q.put(q.o, origins);
+    q.put(q.d, directions);
+    *q.overflow = 0u;
     GiLaunch l = make_launch(ctx, sc);
-    trace_rays(l, sc->view, o.as<float4>(), d.as<float4>(), n, h.as<float4>(), ov.as<uint32_t>(), nullptr, s);
+    trace_rays(l, sc->view, q.o, q.d, n, q.h, q.overflow, nullptr, s);
     OL_HIP_CHECK(hipGetLastError());
     OL_HIP_CHECK(hipStreamSynchronize(s));
-    uint32_t overflow = 0;
-    OL_HIP_CHECK(hipMemcpy(&overflow, ov.ptr, 4, hipMemcpyDeviceToHost));
-    if (overflow) throw OlError{OLHIP_ERR_RUNTIME, "traversal stack overflow"};
-    OL_HIP_CHECK(hipMemcpy(hits, h.ptr, sizeof(float4) * n, hipMemcpyDeviceToHost));
+    if (*q.overflow) throw OlError{OLHIP_ERR_RUNTIME, "traversal stack overflow"};
+    q.get(hits, q.h);
   });
 }
 
@@ -1398,7 +1455,7 @@ int olhip_e0_end(olhip_ctx* ctx, uint32_t samples, float* out_rgba) {
     e0_finish(f.params, f.state, samples, f.out.as<float4>(), s);
     OL_HIP_CHECK(hipGetLastError());
     OL_HIP_CHECK(hipStreamSynchronize(s));
-    OL_HIP_CHECK(hipMemcpy(out_rgba, f.out.ptr, 16ull * f.params.width * f.params.height, hipMemcpyDeviceToHost));
+    ctx->copier->download(out_rgba, f.out.ptr, 16ull * f.params.width * f.params.height);
     f.open = false;
   });
 }

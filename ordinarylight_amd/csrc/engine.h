@@ -27,6 +27,7 @@
 #include "../../include/olhip.h"
 #include "e0.h"
 #include "gi.h"
+#include "hostcopy.h"
 #include "internal.h"
 
 struct olhip_scene {
@@ -82,7 +83,8 @@ class Engine {
   // accumulating) plus the steps still in flight.  Callers hold no lock; the
   // engine serialises steps.
   uint32_t step();
-  void run_until_idle();
+  // `outputs`: destinations of the results, populated while the device works.
+  void run_until_idle(Prefault* outputs = nullptr);
   int state(uint64_t id);
   // Copies the result (optional) and statistics, then forgets the job.
   void take_result(uint64_t id, float* out_rgba, olhip_job_stats* stats, bool keep = false);
@@ -262,6 +264,14 @@ struct olhip_ctx {
   DevBuf image;  // last single frame (olhip_frame_download, olhip_frame_output)
   uint32_t image_pixels = 0, image_width = 0, image_height = 0;
   DevBuf spill;  // olhip_trace
+  // Buffers of olhip_trace and olhip_camera_rays, kept between calls up to a
+  // bound: rays and hits on the device, and pinned memory that the
+  // kernels read and write directly for calls of a few rays.
+  std::mutex query_mu;
+  DevBuf query_o, query_d, query_h;
+  float4* query_host = nullptr;  // origins, directions, hits, then the overflow word
+  // Host copies of images, products, rays and hits.
+  std::unique_ptr<HostCopier> copier;
   // Device address of the fixed traversal spill array (olhip_trace_device).
   uint32_t* trace_scratch = nullptr;
   // Reference-estimator frame.

@@ -7,6 +7,7 @@
 #include <cstring>
 
 #include "engine.h"
+#include "output.h"
 
 // ---- RangeAllocator -------------------------------------------------------------------
 void RangeAllocator::reset(uint64_t size) {
@@ -810,10 +811,10 @@ void Engine::retire_front() {
   }
 }
 
-void Engine::run_until_idle() {
+void Engine::run_until_idle(Prefault* outputs) {
   if (worker_running_) throw OlError{OLHIP_ERR_RUNTIME, "the engine's worker thread is running"};
-  while (step() > 0) {
-  }
+  while (step() > 0)
+    if (outputs) outputs->advance();
 }
 
 int Engine::state(uint64_t id) {
@@ -864,9 +865,8 @@ void Engine::take_result(uint64_t id, float* out_rgba, olhip_job_stats* stats, b
     if (keep) {
       if (out_rgba) {
         OL_HIP_CHECK(hipSetDevice(ctx_->device));
-        OL_HIP_CHECK(hipMemcpy(out_rgba, it->second->image.ptr,
-                               sizeof(float4) * it->second->desc.width * it->second->desc.height,
-                               hipMemcpyDeviceToHost));
+        ctx_->copier->download(out_rgba, it->second->image.ptr,
+                               sizeof(float4) * it->second->desc.width * it->second->desc.height);
       }
       return;
     }
@@ -875,8 +875,7 @@ void Engine::take_result(uint64_t id, float* out_rgba, olhip_job_stats* stats, b
   }
   OL_HIP_CHECK(hipSetDevice(ctx_->device));
   if (out_rgba)
-    OL_HIP_CHECK(hipMemcpy(out_rgba, j->image.ptr, sizeof(float4) * j->desc.width * j->desc.height,
-                           hipMemcpyDeviceToHost));
+    ctx_->copier->download(out_rgba, j->image.ptr, sizeof(float4) * j->desc.width * j->desc.height);
   std::lock_guard<std::mutex> g(mu_);
   keep_buffers(*j);
 }
@@ -891,24 +890,23 @@ void Engine::products(uint64_t id, float* depth, float* normal, uint32_t* primit
   OL_HIP_CHECK(hipSetDevice(ctx_->device));
   if (depth || normal) {
     if (!(j.desc.products & OLHIP_PRODUCT_PRIMARY)) throw OlError{OLHIP_ERR_VALUE, "primary-hit products not requested"};
-    std::vector<float4> g4(np);
-    OL_HIP_CHECK(hipMemcpy(g4.data(), j.geo.ptr, sizeof(float4) * np, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < np; ++i) {
-      if (depth) depth[i] = g4[i].x;
-      if (normal) {
-        normal[3 * i] = g4[i].y;
-        normal[3 * i + 1] = g4[i].z;
-        normal[3 * i + 2] = g4[i].w;
-      }
-    }
+    // The finished job's pixel sums (32 bytes per pixel) are scratch now.
+    float* planes = j.acc.as<float>();
+    float* normals = planes + (np + 3) / 4 * 4;
+    launch_split_primary(j.geo.as<float4>(), (uint32_t)np, depth ? planes : nullptr, normal ? normals : nullptr,
+                         ctx_->stream);
+    OL_HIP_CHECK(hipGetLastError());
+    OL_HIP_CHECK(hipStreamSynchronize(ctx_->stream));
+    if (depth) ctx_->copier->download(depth, planes, sizeof(float) * np);
+    if (normal) ctx_->copier->download(normal, normals, sizeof(float) * 3 * np);
   }
   if (primitive) {
     if (!(j.desc.products & OLHIP_PRODUCT_PRIMARY)) throw OlError{OLHIP_ERR_VALUE, "primary-hit products not requested"};
-    OL_HIP_CHECK(hipMemcpy(primitive, j.prim.ptr, sizeof(uint32_t) * np, hipMemcpyDeviceToHost));
+    ctx_->copier->download(primitive, j.prim.ptr, sizeof(uint32_t) * np);
   }
   if (variance) {
     if (!(j.desc.products & OLHIP_PRODUCT_VARIANCE)) throw OlError{OLHIP_ERR_VALUE, "variance not requested"};
-    OL_HIP_CHECK(hipMemcpy(variance, j.variance.ptr, sizeof(float) * np, hipMemcpyDeviceToHost));
+    ctx_->copier->download(variance, j.variance.ptr, sizeof(float) * np);
   }
 }
 

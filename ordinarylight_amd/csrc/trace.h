@@ -193,7 +193,8 @@ struct TravStack {
     } else if (sp - LSTACK < spill_cap) {
       spill[(sp - LSTACK) * spill_stride] = v;
     } else {
-      atomicOr(overflow, 1u);
+      // A plain store (every lane's is the same): the word may be host memory.
+      *overflow = 1u;
       return;
     }
     ++sp;
