@@ -29,27 +29,55 @@ OL_DEV float wrap_coordinate(float v, uint32_t mode) {
 OL_DEV int wrap_index(int v, int size, uint32_t mode) {
   if (mode == 1u) return min(max(v, 0), size - 1);
   const int period = mode == 2u ? size * 2 : size;
-  int w = v % period;
-  if (w < 0) w += period;
+  // A wrapped coordinate's texels lie at most one period off, so the
+  // remainder is one conditional step; the division only serves the rest (a
+  // texture of one texel, a coordinate that rounded up).
+  int w = v < 0 ? v + period : (v >= period ? v - period : v);
+  if (w < 0 || w >= period) {
+    w = v % period;
+    if (w < 0) w += period;
+  }
   if (mode == 2u && w >= size) return period - 1 - w;
   return w;
 }
 
-OL_DEV float4 decode_texel(uint32_t word, bool srgb) {
-  float4 c = make_float4((float)(word & 255u) / 255.0f, (float)((word >> 8) & 255u) / 255.0f,
-                         (float)((word >> 16) & 255u) / 255.0f, (float)(word >> 24) / 255.0f);
-  if (srgb) {
-    c.x = srgb_channel(c.x);
-    c.y = srgb_channel(c.y);
-    c.z = srgb_channel(c.z);
+// Texel decoding: by computation, or from a table of the 256 linear and the
+// 256 sRGB channel values that a block has computed the same way
+// (fill_channel_table).
+struct DecodeTexel {
+  OL_DEV float4 operator()(uint32_t word, bool srgb) const {
+    float4 c = make_float4((float)(word & 255u) / 255.0f, (float)((word >> 8) & 255u) / 255.0f,
+                           (float)((word >> 16) & 255u) / 255.0f, (float)(word >> 24) / 255.0f);
+    if (srgb) {
+      c.x = srgb_channel(c.x);
+      c.y = srgb_channel(c.y);
+      c.z = srgb_channel(c.z);
+    }
+    return c;
   }
-  return c;
+};
+constexpr uint32_t kChannelTable = 512;
+struct LookUpTexel {
+  const float* table;
+  OL_DEV float4 operator()(uint32_t word, bool srgb) const {
+    const float* rgb = table + (srgb ? 256 : 0);
+    return make_float4(rgb[word & 255u], rgb[(word >> 8) & 255u], rgb[(word >> 16) & 255u], table[word >> 24]);
+  }
+};
+OL_DEV void fill_channel_table(float* table) {
+  for (uint32_t k = threadIdx.x; k < 256u; k += blockDim.x) {
+    const float v = (float)k / 255.0f;
+    table[k] = v;
+    table[256u + k] = srgb_channel(v);
+  }
+  __syncthreads();
 }
 
+template <class Decode>
 OL_DEV float4 fetch_texel(const uint32_t* words, uint32_t offset, int w, int h, int x, int y, uint32_t wrap_x,
-                          uint32_t wrap_y, bool srgb) {
+                          uint32_t wrap_y, bool srgb, Decode decode) {
   const int xx = wrap_index(x, w, wrap_x), yy = wrap_index(y, h, wrap_y);
-  return decode_texel(words[offset + (uint32_t)(yy * w + xx)], srgb);
+  return decode(words[offset + (uint32_t)(yy * w + xx)], srgb);
 }
 
 OL_DEV float4 mix4(float4 a, float4 b, float t) {
@@ -58,8 +86,9 @@ OL_DEV float4 mix4(float4 a, float4 b, float t) {
 }
 
 // One mip level, nearest or bilinear (shadeSampleTextureLevel).
+template <class Decode>
 OL_DEV float4 sample_level(const uint32_t* words, uint32_t base, int bw, int bh, uint32_t level, float u, float v,
-                           uint32_t wrap_x, uint32_t wrap_y, bool srgb, bool linear) {
+                           uint32_t wrap_x, uint32_t wrap_y, bool srgb, bool linear, Decode decode) {
   uint32_t offset = base;
   int w = bw, h = bh;
   for (uint32_t k = 0; k < level && k < 32u; ++k) {
@@ -70,23 +99,24 @@ OL_DEV float4 sample_level(const uint32_t* words, uint32_t base, int bw, int bh,
   const float wu = wrap_coordinate(u, wrap_x), wv = wrap_coordinate(v, wrap_y);
   if (!linear) {
     return fetch_texel(words, offset, w, h, (int)floorf(wu * (float)w), (int)floorf(wv * (float)h), wrap_x, wrap_y,
-                       srgb);
+                       srgb, decode);
   }
   const float tx = wu * (float)w - 0.5f, ty = wv * (float)h - 0.5f;
   const int x0 = (int)floorf(tx), y0 = (int)floorf(ty);
   const float fx = tx - floorf(tx), fy = ty - floorf(ty);
-  const float4 top = mix4(fetch_texel(words, offset, w, h, x0, y0, wrap_x, wrap_y, srgb),
-                          fetch_texel(words, offset, w, h, x0 + 1, y0, wrap_x, wrap_y, srgb), fx);
-  const float4 bottom = mix4(fetch_texel(words, offset, w, h, x0, y0 + 1, wrap_x, wrap_y, srgb),
-                             fetch_texel(words, offset, w, h, x0 + 1, y0 + 1, wrap_x, wrap_y, srgb), fx);
+  const float4 top = mix4(fetch_texel(words, offset, w, h, x0, y0, wrap_x, wrap_y, srgb, decode),
+                          fetch_texel(words, offset, w, h, x0 + 1, y0, wrap_x, wrap_y, srgb, decode), fx);
+  const float4 bottom = mix4(fetch_texel(words, offset, w, h, x0, y0 + 1, wrap_x, wrap_y, srgb, decode),
+                             fetch_texel(words, offset, w, h, x0 + 1, y0 + 1, wrap_x, wrap_y, srgb, decode), fx);
   return mix4(top, bottom, fy);
 }
 
 // A material texture through its binding: transform, mip level from the
 // footprint, trilinear blend (shadeSampleMaterialTexture).  White when the
 // binding is absent.
+template <class Decode>
 OL_DEV float4 sample_material_texture(const DScene& sc, float binding_value, float u0, float v0, float u1, float v1,
-                                      bool srgb, float fp0, float fp1) {
+                                      bool srgb, float fp0, float fp1, Decode decode) {
   const int b = (int)binding_value;
   if (b < 0) return make_float4(1.0f, 1.0f, 1.0f, 1.0f);
   const float4 r0 = sc.bindings[2 * b], r1 = sc.bindings[2 * b + 1];
@@ -108,9 +138,9 @@ OL_DEV float4 sample_material_texture(const DScene& sc, float binding_value, flo
   const float lod = fminf(fmaxf(log2f(fmaxf(fp * (float)max(w, h), 1.0f)), 0.0f), (float)(max(levels, 1u) - 1u));
   const uint32_t lower = (uint32_t)floorf(lod);
   const bool linear = (flags & 16u) != 0u;
-  const float4 first = sample_level(sc.tex_words, offset, w, h, lower, u, v, wx, wy, srgb, linear);
+  const float4 first = sample_level(sc.tex_words, offset, w, h, lower, u, v, wx, wy, srgb, linear, decode);
   if (!linear || lower + 1u >= levels) return first;
-  const float4 second = sample_level(sc.tex_words, offset, w, h, lower + 1u, u, v, wx, wy, srgb, true);
+  const float4 second = sample_level(sc.tex_words, offset, w, h, lower + 1u, u, v, wx, wy, srgb, true, decode);
   return mix4(first, second, lod - floorf(lod));
 }
 
@@ -128,7 +158,7 @@ OL_DEV f3 environment_image(const DScene& sc, f3 d) {
     const uint32_t flags = sc.tex_words[meta + 4u];
     const float4 c = sample_level(sc.tex_words, sc.tex_words[meta + 1u], (int)sc.tex_words[meta + 2u],
                                   (int)sc.tex_words[meta + 3u], 0u, u, v, flags & 3u, (flags >> 2) & 3u, false,
-                                  (flags & 16u) != 0u);
+                                  (flags & 16u) != 0u, DecodeTexel{});
     enc = mk3(c.x, c.y, c.z);
   }
   const f3 rad = mk3(exp2f(enc.x * sc.env_log_range) - 1.0f, exp2f(enc.y * sc.env_log_range) - 1.0f,
