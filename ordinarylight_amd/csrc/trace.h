@@ -5,8 +5,8 @@
 // lds[k * BLOCK + t], bank-conflict free), deeper entries spill to a per-lane
 // column of a global buffer.  The total depth is chosen on the host from the
 // BVH's level count (a 4-wide level leaves at most three entries, and four
-// are pushed before the next is taken), so it cannot overflow; the small LDS part keeps occupancy bounded by registers,
-// not LDS.
+// are pushed before the next is taken), so it cannot overflow; the small LDS
+// part keeps occupancy bounded by registers, not LDS.
 //
 // Closest-hit semantics are those of a ray query over opaque triangles
 // (native_intersection.glsl:44-183): candidates with tmin <= t <= tmax; the
