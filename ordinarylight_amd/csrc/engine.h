@@ -87,8 +87,10 @@ class Engine {
   void run_until_idle(Prefault* outputs = nullptr);
   int state(uint64_t id);
   // Copies the result (optional) and statistics, then forgets the job.
-  void take_result(uint64_t id, float* out_rgba, olhip_job_stats* stats, bool keep = false);
-  // Copies a done job's products (any pointer may be null).
+  void take_result(uint64_t id, float* out_rgba, olhip_job_stats* stats);
+  // Copies a done job's products (any pointer may be null).  Touches neither
+  // the engine's stream, which a running worker may be capturing, nor holds
+  // a lock while it copies.
   void products(uint64_t id, float* depth, float* normal, uint32_t* primitive, float* variance);
   void engine_stats(olhip_engine_stats* out);
   // Device image of a done job (valid until take_result).
@@ -140,7 +142,8 @@ class Engine {
     std::vector<Chunk> resident, finished;
     uint32_t passed = 0;        // admission rounds in which this job did not fit
     int status = OLHIP_JOB_QUEUED;
-    DevBuf acc, image, geo, prim, lum, variance, res, surf;
+    uint32_t readers = 0;       // products() calls copying from its buffers (take_result waits for them)
+    DevBuf acc, image, depth, normal, prim, lum, variance, res, surf;
     olhip_job_stats stats{};
     std::string error;
   };

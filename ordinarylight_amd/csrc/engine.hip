@@ -7,7 +7,6 @@
 #include <cstring>
 
 #include "engine.h"
-#include "output.h"
 
 // ---- RangeAllocator -------------------------------------------------------------------
 void RangeAllocator::reset(uint64_t size) {
@@ -354,7 +353,8 @@ bool Engine::admit(Job& j, int slot) {
         take_buffer(j.acc, sizeof(double4) * np);
         take_buffer(j.image, sizeof(float4) * np);
         if (d.products & OLHIP_PRODUCT_PRIMARY) {
-          take_buffer(j.geo, sizeof(float4) * np);
+          take_buffer(j.depth, sizeof(float) * np);
+          take_buffer(j.normal, sizeof(float) * 3 * np);
           take_buffer(j.prim, sizeof(uint32_t) * np);
         }
         if (d.products & OLHIP_PRODUCT_VARIANCE) {
@@ -381,7 +381,8 @@ bool Engine::admit(Job& j, int slot) {
         J.surf_in = j.surf.as<float4>() + ((pass + 1u) & 1u) * 2 * np;
       }
       j.buffers = true;
-      J.geo = (d.products & OLHIP_PRODUCT_PRIMARY) ? j.geo.as<float4>() : nullptr;
+      J.depth = (d.products & OLHIP_PRODUCT_PRIMARY) ? j.depth.as<float>() : nullptr;
+      J.normal = (d.products & OLHIP_PRODUCT_PRIMARY) ? j.normal.as<float>() : nullptr;
       J.prim = (d.products & OLHIP_PRODUCT_PRIMARY) ? j.prim.as<uint32_t>() : nullptr;
       j.status = OLHIP_JOB_RUNNING;
       ++j.stats.chunks;
@@ -436,7 +437,7 @@ void Engine::take_buffer(DevBuf& dst, size_t bytes) {
 // has completed (no queued work uses the buffers).
 void Engine::keep_buffers(Job& j) {
   std::lock_guard<std::mutex> g(ctx_->spare_mu);
-  for (DevBuf* b : {&j.acc, &j.image, &j.geo, &j.prim, &j.lum, &j.variance, &j.res, &j.surf}) {
+  for (DevBuf* b : {&j.acc, &j.image, &j.depth, &j.normal, &j.prim, &j.lum, &j.variance, &j.res, &j.surf}) {
     if (!b->ptr) continue;
     ctx_->spare_bytes += b->bytes;
     ctx_->spare.push_back(std::move(*b));
@@ -849,11 +850,15 @@ const float4* Engine::device_image(uint64_t id) {
   return it->second->image.as<float4>();
 }
 
-void Engine::take_result(uint64_t id, float* out_rgba, olhip_job_stats* stats, bool keep) {
+void Engine::take_result(uint64_t id, float* out_rgba, olhip_job_stats* stats) {
   std::unique_ptr<Job> j;
   {
-    std::lock_guard<std::mutex> g(mu_);
+    std::unique_lock<std::mutex> lk(mu_);
     auto it = jobs_.find(id);
+    while (it != jobs_.end() && it->second->readers != 0) {
+      cv_.wait(lk);
+      it = jobs_.find(id);
+    }
     if (it == jobs_.end()) throw OlError{OLHIP_ERR_VALUE, "unknown job id"};
     if (it->second->status == OLHIP_JOB_FAILED) {
       std::string e = it->second->error;
@@ -862,14 +867,6 @@ void Engine::take_result(uint64_t id, float* out_rgba, olhip_job_stats* stats, b
     }
     if (it->second->status != OLHIP_JOB_DONE) throw OlError{OLHIP_ERR_RUNTIME, "job is not done"};
     if (stats) *stats = it->second->stats;
-    if (keep) {
-      if (out_rgba) {
-        OL_HIP_CHECK(hipSetDevice(ctx_->device));
-        ctx_->copier->download(out_rgba, it->second->image.ptr,
-                               sizeof(float4) * it->second->desc.width * it->second->desc.height);
-      }
-      return;
-    }
     j = std::move(it->second);
     jobs_.erase(it);
   }
@@ -881,33 +878,34 @@ void Engine::take_result(uint64_t id, float* out_rgba, olhip_job_stats* stats, b
 }
 
 void Engine::products(uint64_t id, float* depth, float* normal, uint32_t* primitive, float* variance) {
-  std::lock_guard<std::mutex> g(mu_);
-  auto it = jobs_.find(id);
-  if (it == jobs_.end()) throw OlError{OLHIP_ERR_VALUE, "unknown job id"};
-  const Job& j = *it->second;
-  if (j.status != OLHIP_JOB_DONE) throw OlError{OLHIP_ERR_RUNTIME, "job is not done"};
-  const size_t np = (size_t)j.desc.width * j.desc.height;
+  Job* j = nullptr;
+  {
+    std::lock_guard<std::mutex> g(mu_);
+    auto it = jobs_.find(id);
+    if (it == jobs_.end()) throw OlError{OLHIP_ERR_VALUE, "unknown job id"};
+    j = it->second.get();
+    if (j->status != OLHIP_JOB_DONE) throw OlError{OLHIP_ERR_RUNTIME, "job is not done"};
+    if ((depth || normal || primitive) && !(j->desc.products & OLHIP_PRODUCT_PRIMARY))
+      throw OlError{OLHIP_ERR_VALUE, "primary-hit products not requested"};
+    if (variance && !(j->desc.products & OLHIP_PRODUCT_VARIANCE))
+      throw OlError{OLHIP_ERR_VALUE, "variance not requested"};
+    ++j->readers;
+  }
+  struct Reading {
+    Engine& engine;
+    Job& job;
+    ~Reading() {
+      std::lock_guard<std::mutex> g(engine.mu_);
+      --job.readers;
+      engine.cv_.notify_all();
+    }
+  } reading{*this, *j};
   OL_HIP_CHECK(hipSetDevice(ctx_->device));
-  if (depth || normal) {
-    if (!(j.desc.products & OLHIP_PRODUCT_PRIMARY)) throw OlError{OLHIP_ERR_VALUE, "primary-hit products not requested"};
-    // The finished job's pixel sums (32 bytes per pixel) are scratch now.
-    float* planes = j.acc.as<float>();
-    float* normals = planes + (np + 3) / 4 * 4;
-    launch_split_primary(j.geo.as<float4>(), (uint32_t)np, depth ? planes : nullptr, normal ? normals : nullptr,
-                         ctx_->stream);
-    OL_HIP_CHECK(hipGetLastError());
-    OL_HIP_CHECK(hipStreamSynchronize(ctx_->stream));
-    if (depth) ctx_->copier->download(depth, planes, sizeof(float) * np);
-    if (normal) ctx_->copier->download(normal, normals, sizeof(float) * 3 * np);
-  }
-  if (primitive) {
-    if (!(j.desc.products & OLHIP_PRODUCT_PRIMARY)) throw OlError{OLHIP_ERR_VALUE, "primary-hit products not requested"};
-    ctx_->copier->download(primitive, j.prim.ptr, sizeof(uint32_t) * np);
-  }
-  if (variance) {
-    if (!(j.desc.products & OLHIP_PRODUCT_VARIANCE)) throw OlError{OLHIP_ERR_VALUE, "variance not requested"};
-    ctx_->copier->download(variance, j.variance.ptr, sizeof(float) * np);
-  }
+  const size_t plane = sizeof(float) * j->desc.width * j->desc.height;
+  if (depth) ctx_->copier->download(depth, j->depth.ptr, plane);
+  if (normal) ctx_->copier->download(normal, j->normal.ptr, 3 * plane);
+  if (primitive) ctx_->copier->download(primitive, j->prim.ptr, plane);
+  if (variance) ctx_->copier->download(variance, j->variance.ptr, plane);
 }
 
 void Engine::engine_stats(olhip_engine_stats* out) {

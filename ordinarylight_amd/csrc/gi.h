@@ -108,10 +108,12 @@ struct JobDev {
   uint32_t eseg;     // shadow-entry slots per segment
   uint32_t append;   // continuations / shadow groups a segment accepts per step (<= seg)
   uint32_t pad;
-  // Primary-hit products of sample 0 (null unless requested): per pixel
-  // (t or +inf, geometric normal) and the original triangle index (or
-  // OL_NONE) (wavefront_intersect.comp:317-356, targets/vulkan/core.py:4500-4536).
-  float4* geo;
+  // Primary-hit products of sample 0 (null unless requested), each the plane
+  // the caller gets: distance (or +inf), geometric normal (3 floats a pixel)
+  // and original triangle index (or OL_NONE) (wavefront_intersect.comp:317-356,
+  // targets/vulkan/core.py:4500-4536).
+  float* depth;
+  float* normal;
   uint32_t* prim;
   // ReSTIR DI (null unless enabled): this pass's and the previous pass's
   // stored reservoirs and primary surfaces (2 x float4 per pixel: shading

@@ -1385,6 +1385,17 @@ k_restir(Wave W, uint32_t in, uint32_t gen) {
   }
 }
 
+// A primary hit into the job's product planes, in the layout that the caller
+// gets, so that a download is a copy and nothing has to run once the job is
+// done (the engine's stream belongs to its steps, and may be under capture).
+OL_DEV void put_primary(const JobDev& J, uint32_t pixel, float t, f3 n, uint32_t prim) {
+  J.depth[pixel] = t;
+  J.normal[3u * pixel] = n.x;
+  J.normal[3u * pixel + 1u] = n.y;
+  J.normal[3u * pixel + 2u] = n.z;
+  J.prim[pixel] = prim;
+}
+
 // ---- shade -----------------------------------------------------------------------------------
 // One wave per 64-ray chunk (grid-stride over chunks), so the job and its
 // parameters are wave-uniform.  Outputs go to the job's segment
@@ -1433,12 +1444,11 @@ OL_DEV void shade_chunk(const Wave& W, uint32_t in, uint32_t gen, const ChunkLoc
           break;
         }
         // Sample 0's primary hit for the named products.
-        const bool record_primary = J.geo != nullptr && T.w == 0.0f && P.sample_base == 0u &&
+        const bool record_primary = J.depth != nullptr && T.w == 0.0f && P.sample_base == 0u &&
                                     path - J.base < P.width * P.height;
         if (slot == OL_NONE) {
           if (record_primary) {
-            J.geo[M.x] = make_float4(__builtin_huge_valf(), 0.0f, 0.0f, 0.0f);
-            J.prim[M.x] = OL_NONE;
+            put_primary(J, M.x, __builtin_huge_valf(), mk3(0.0f, 0.0f, 0.0f), OL_NONE);
           }
           // shadeResolveEnvironmentMiss
           f3 env = environment_radiance(sc, incoming);
@@ -1464,8 +1474,7 @@ OL_DEV void shade_chunk(const Wave& W, uint32_t in, uint32_t gen, const ChunkLoc
         resolve_surface(W, sc, i, slot, ro, rd, hv, hitp, gn, nrm, cw, prim, mat_id, entering);
         if (W.work) count_active(&W.work[6]);
         if (record_primary) {
-          J.geo[M.x] = make_float4(t, gn.x, gn.y, gn.z);
-          J.prim[M.x] = prim;
+          put_primary(J, M.x, t, gn, prim);
         }
         Mat mat = load_mat(sc.materials, mat_id);
         if (sc.face) apply_face(sc, slot, mat);

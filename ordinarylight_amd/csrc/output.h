@@ -12,10 +12,6 @@ constexpr uint32_t kOutputRgba8 = 0, kOutputNv12 = 1, kOutputP010 = 2;
 // pitch = 2 * width bytes; the chroma plane follows the luma plane).
 size_t output_bytes(uint32_t format, uint32_t width, uint32_t height);
 
-// Splits primary-hit records (distance, normal) into a plane of distances and
-// one of normals (3 floats per pixel); either may be null.
-void launch_split_primary(const float4* geo, uint32_t n, float* depth, float* normal, hipStream_t st);
-
 // Writes the frame: RGBA8 and NV12 take a width x height HDR image
 // (src_w == width, src_h == height); P010 scales src_w x src_h to width x
 // height by nearest neighbour.  NV12 and P010 need width % 4 == 0 and even

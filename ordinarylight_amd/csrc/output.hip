@@ -123,25 +123,6 @@ __global__ void __launch_bounds__(256) k_p010(const float4* __restrict__ hdr, ui
                   ((ten_bit_value(512.0f + 896.0f * cr709(second)) << 6) << 16);
 }
 
-// 16 bytes read and 16 written per pixel, all coalesced (the host did this
-// pixel by pixel on one thread).
-__global__ void __launch_bounds__(256) k_split_primary(const float4* __restrict__ geo, uint32_t n,
-                                                       float* __restrict__ depth, float* __restrict__ normal) {
-  __shared__ float rows[3 * 256];
-  const uint32_t first = blockIdx.x * 256u, i = first + threadIdx.x;
-  if (i < n) {
-    const float4 g = geo[i];
-    if (depth) depth[i] = g.x;
-    rows[3u * threadIdx.x] = g.y;
-    rows[3u * threadIdx.x + 1u] = g.z;
-    rows[3u * threadIdx.x + 2u] = g.w;
-  }
-  __syncthreads();
-  if (!normal) return;
-  const uint32_t words = 3u * min(256u, n - first);
-  for (uint32_t k = threadIdx.x; k < words; k += 256u) normal[3ull * first + k] = rows[k];
-}
-
 }  // namespace
 
 size_t output_bytes(uint32_t format, uint32_t width, uint32_t height) {
@@ -163,9 +144,4 @@ void launch_output(uint32_t format, const float4* hdr, uint32_t src_w, uint32_t 
     const dim3 grid((width / 4u + 255u) / 256u, height / 2u);
     hipLaunchKernelGGL(k_p010, grid, dim3(256), 0, st, hdr, src_w, src_h, width, height, 2u * width, exposure, out);
   }
-}
-
-void launch_split_primary(const float4* geo, uint32_t n, float* depth, float* normal, hipStream_t st) {
-  if (n == 0) return;
-  hipLaunchKernelGGL(k_split_primary, dim3((n + 255u) / 256u), dim3(256), 0, st, geo, n, depth, normal);
 }
