@@ -12,7 +12,9 @@
  * MemoryError); olhip_last_error() describes the last failure of the calling
  * thread.  Pointers are plain host pointers; nothing here takes ownership of
  * caller memory.  One context owns one HIP stream on one device; calls on
- * one context must not overlap.
+ * one context must not overlap, apart from those marked thread-safe (an
+ * engine's running worker is no call: scenes may be built and rays traced
+ * beside it).
  */
 #ifndef OLHIP_H
 #define OLHIP_H

@@ -158,7 +158,7 @@ class Engine {
   static constexpr uint32_t kKeyAcc = 64u, kKeyGen = 128u, kKeyFused = 256u;
   hipGraphExec_t graph_for(uint32_t key);
   void clear_graphs();
-  void launch_step(uint32_t key, bool timed, int buf);
+  void launch_step(uint32_t key, bool timed, int buf, hipStream_t s);
   // A step queued on the stream whose report has not been applied yet.
   struct InFlight {
     uint64_t seq = 0;
@@ -218,6 +218,10 @@ class Engine {
   bool profiling_ = false;
   std::unordered_map<uint32_t, hipGraphExec_t> graphs_;  // by step_key
   bool graph_valid_ = false;
+  // Step graphs are captured here: the context's stream stays usable by other
+  // threads (a scene built or rays traced while the worker meets a new step
+  // shape would otherwise be recorded into that step's graph).
+  hipStream_t capture_ = nullptr;
   // Job table (host copy; the device copy is refreshed when it changes) and
   // pinned staging, one set per in-flight step.
   std::vector<JobDev> jobs_state_;

@@ -115,6 +115,7 @@ Engine::Engine(olhip_ctx* ctx, const olhip_engine_config& cfg) : ctx_(ctx), cfg_
     stage_host_[b] = pinned<StepStage>(1);
     report_host_[b] = pinned<uint32_t>(C_WORDS - C_OVERFLOW);
   }
+  if (cfg_.use_graph) OL_HIP_CHECK(hipStreamCreateWithFlags(&capture_, hipStreamNonBlocking));
   OL_HIP_CHECK(hipEventCreate(&begin_));
   for (hipEvent_t& e : done_) OL_HIP_CHECK(hipEventCreate(&e));
   t0_ms_ = 0;
@@ -137,6 +138,7 @@ Engine::~Engine() {
   // Jobs never taken leave their buffers to the context's pool.
   for (auto& kv : jobs_) keep_buffers(*kv.second);
   for (auto& kv : graphs_) (void)hipGraphExecDestroy(kv.second);
+  if (capture_) (void)hipStreamDestroy(capture_);
   if (begin_) (void)hipEventDestroy(begin_);
   for (hipEvent_t e : done_)
     if (e) (void)hipEventDestroy(e);
@@ -468,8 +470,7 @@ void Engine::drop_chunks(Job& j) {
   acc_jobs_.erase(std::remove(acc_jobs_.begin(), acc_jobs_.end(), j.id), acc_jobs_.end());
 }
 
-void Engine::launch_step(uint32_t key, bool timed, int buf) {
-  hipStream_t s = ctx_->stream;
+void Engine::launch_step(uint32_t key, bool timed, int buf, hipStream_t s) {
   const uint32_t in = key & 1u, kinds = (key >> 1) & kStepKinds;
   const bool gen = (key & kKeyGen) != 0u;
   if (key & kKeyAcc) wave_accumulate(wave_, ctx_->cu_count, s);
@@ -515,18 +516,17 @@ hipGraphExec_t Engine::graph_for(uint32_t key) {
   if (!graph_valid_) clear_graphs();
   auto it = graphs_.find(key);
   if (it != graphs_.end()) return it->second;
-  hipStream_t s = ctx_->stream;
   hipGraph_t g = nullptr;
   quiesce();
-  OL_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+  OL_HIP_CHECK(hipStreamBeginCapture(capture_, hipStreamCaptureModeThreadLocal));
   try {
-    launch_step(key, false, 0);
+    launch_step(key, false, 0, capture_);
   } catch (...) {
-    (void)hipStreamEndCapture(s, &g);
+    (void)hipStreamEndCapture(capture_, &g);
     if (g) (void)hipGraphDestroy(g);
     throw;
   }
-  OL_HIP_CHECK(hipStreamEndCapture(s, &g));
+  OL_HIP_CHECK(hipStreamEndCapture(capture_, &g));
   hipGraphExec_t exec = nullptr;
   OL_HIP_CHECK(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0));
   OL_HIP_CHECK(hipGraphDestroy(g));
@@ -700,7 +700,7 @@ bool Engine::launch_next() {
     // Only accumulation left: no traversal launches.
     wave_accumulate(wave_, ctx_->cu_count, s);
   } else if (profiling_ || !cfg_.use_graph || seq_ == 0) {
-    launch_step(key, profiling_, b);
+    launch_step(key, profiling_, b, s);
   } else {
     OL_HIP_CHECK(hipGraphLaunch(graph_for(key), s));
   }

@@ -105,3 +105,50 @@ def test_products_while_the_worker_meets_new_step_shapes(ctx, scenes, graph):
                 assert np.array_equal(image, want[id(j)][1])
             for j, k in zip(early, ids):
                 assert np.array_equal(engine.result(k)[0], want[id(j)][1])
+
+
+def test_scenes_and_rays_while_the_worker_meets_new_step_shapes(ctx, scenes):
+    """A scene built and rays traced on the worker's context, while it captures
+    step shapes, give what they give alone, and so do the worker's images."""
+    built, _ = workloads.tessellated_room(5, 3000)
+    rng = np.random.default_rng(1)
+    o = rng.uniform(-1.0, 1.0, (5000, 3)).astype(np.float32)
+    d = rng.normal(size=o.shape).astype(np.float32)
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+
+    def build_and_trace():
+        ds = DeviceScene(ctx, built, 2)
+        try:
+            nodes, tri = ds.bvh_arrays()
+            return [nodes, tri.view(np.uint32), *ds.trace(o, d, 0.001, 1e30), *ds.trace(o[:100], d[:100], 0.001, 1e30)]
+        finally:
+            ds.close()
+
+    want = build_and_trace()
+    jobs = [Job(*scenes[key], w, h, samples, 0, HipRendererConfig(max_bounces=bounces, **options), products=3)
+            for key, w, h, samples, bounces, options in (
+                ("room", 97, 65, 3, 3, {}), ("inst", 96, 64, 2, 5, {}), ("textured", 80, 60, 3, 4, {}),
+                ("inst", 64, 64, 3, 4, {"wavefront_restir_di": True, "wavefront_restir_candidates": 8}),
+                ("textured", 128, 72, 1, 2, {}))]
+    images = [alone(ctx, j)[1] for j in jobs]
+    for _ in range(4):
+        with BatchEngine(ctx, EngineSettings(path_slots=1 << 20)) as engine:
+            engine.start()
+            done, failures = [], []
+
+            def feed():
+                try:
+                    for j in jobs:
+                        k = engine.submit(j)
+                        assert engine.wait(k, 60) == N.JOB_DONE
+                        done.append(engine.result(k)[0])
+                except BaseException as e:  # noqa: BLE001 - reported by the main thread
+                    failures.append(e)
+
+            feeder = threading.Thread(target=feed)
+            feeder.start()
+            while feeder.is_alive():
+                assert all(np.array_equal(a, b) for a, b in zip(build_and_trace(), want))
+            feeder.join()
+            assert not failures, failures
+            assert all(np.array_equal(a, b) for a, b in zip(done, images))
