@@ -4,21 +4,27 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
-#include <cstdint>
 #include <mutex>
 #include <vector>
 
-// A download runs in pieces: a kernel writes a piece into a slot of a pinned
-// ring and raises a flag per 256 KB, and the caller copies each flagged part
-// into the user's memory while the rest is on its way.  The link takes 54 GB/s
-// from the kernel (33 MB in 0.62 ms), one host thread copies 50-80 GB/s
-// between mapped pages.  Copies by the copy engine with an event each took
-// 35 us per MB in pieces of 1 MB, a pageable hipMemcpy 55 us per MB warm; with
-// the page faults of a fresh destination it took 100-220 us per MB, 2.7 ms of
-// a 9.1 ms frame.  Pages are therefore populated by one call per part (27-66
-// us per MB), or beforehand where the caller knows its destination while the
-// device still works (Prefault).
-// Downloads of one HostCopier run one after the other; it holds kRing bytes of
+// A download runs in pieces: the copy engine brings one into a slot of a
+// pinned ring while the caller copies the one before into the user's memory.
+//
+// The copy engine and not a kernel: a kernel fills the link better (33 MB into
+// mapped pages in 1.0-1.2 ms, the copy engine in 1.4, a pageable hipMemcpy in
+// 1.8), but its blocks wait for room beside a worker's traversal waves, which
+// live as long as their launch: a 1 MB image fetched beside a rendering worker
+// took 0.7 ms at the median and 11 ms at worst, here 0.1 and 0.2.
+// Pieces are awaited by synchronising the ring's stream, which follows the
+// copy itself.  An event would go through the stream's hardware queue, which
+// may be the one that a worker's steps use (there are four per process): each
+// piece then waited for a step, 33 MB for 130 ms.
+// Two pieces of 768 KB: 5 MB in 0.17 ms, 33 MB in 1.40 ms into mapped pages
+// and 1.94 into fresh ones; 256 KB 0.26, 1.66 and 2.54, 1 MB 0.21, 1.29 and 2.39.
+// Pages of a fresh destination are populated by one call per part (27-66 us per
+// MB, page faults take 100-220), or beforehand where the caller knows its
+// destination while the device still works (Prefault).
+// Downloads of one HostCopier run one after the other; it holds 1.5 MB of
 // pinned memory, made at its first download.
 class HostCopier {
  public:
@@ -33,16 +39,14 @@ class HostCopier {
   static void prefault(void* dst, size_t bytes);
 
  private:
+  static constexpr size_t kPiece = size_t(768) << 10;
+
   void prepare();
-  void await(const uint32_t* flag, uint32_t value);
 
   int device_;
   std::mutex use_;  // one download at a time
   hipStream_t stream_ = nullptr;
-  char* ring_ = nullptr;               // kSlots pieces
-  uint32_t* flags_ = nullptr;          // pinned: per slot and part, the number of the piece that filled it
-  uint32_t* arrived_ = nullptr;        // device: per slot and part, blocks done
-  uint32_t piece_ = 0;                 // pieces issued so far (never 0 in a flag)
+  char* ring_ = nullptr;  // two pieces
 };
 
 // Populates destinations piece by piece while their data is being computed.

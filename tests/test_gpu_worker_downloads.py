@@ -1,6 +1,7 @@
 """Downloads of finished jobs while the engine's worker renders others."""
 
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -152,3 +153,45 @@ def test_scenes_and_rays_while_the_worker_meets_new_step_shapes(ctx, scenes):
             feeder.join()
             assert not failures, failures
             assert all(np.array_equal(a, b) for a, b in zip(done, images))
+
+
+@pytest.mark.parametrize("streams", range(4))
+def test_a_result_does_not_wait_for_the_worker(hip_device, streams):
+    """A finished image comes back beside a rendering worker about as fast as
+    from an idle device: its copy neither needs compute units nor queues up
+    behind the worker's steps, whichever of the process's four hardware queues
+    the streams share (`streams`: contexts made before, one stream each)."""
+    others = [DeviceContext(hip_device) for _ in range(streams)]
+    ctx = DeviceContext(hip_device)
+    heavy, heavy_cam = workloads.instanced_spheres(1, instances=2000, emitters=2000)
+    light, light_cam = workloads.tessellated_room(1, 2000)
+    heavy_scene, light_scene = DeviceScene(ctx, heavy, 2), DeviceScene(ctx, light, 2)
+    with BatchEngine(ctx, EngineSettings(path_slots=1 << 24)) as engine:
+        done = [engine.submit(Job(light_scene, light_cam, 512, 512, max_bounces=1)) for _ in range(64)]
+        engine.run()
+
+        frames = []
+
+        def fetch(count, pause, worker):
+            took = []
+            for _ in range(count):
+                while worker and sum(engine.poll(k) != N.JOB_DONE for k in frames[-4:]) < 3:
+                    frames.append(engine.submit(Job(heavy_scene, heavy_cam, 1920, 1080, 4, 0, max_bounces=16)))
+                time.sleep(pause)
+                begin = time.perf_counter()
+                engine.result(done.pop())
+                took.append(time.perf_counter() - begin)
+            return sorted(took)[int(0.9 * count)]
+
+        fetch(8, 0.0, False)
+        idle = fetch(16, 0.002, False)
+        engine.start()
+        fetch(4, 0.05, True)
+        busy = fetch(32, 0.003, True)
+        for k in frames:
+            assert engine.wait(k, 60) == N.JOB_DONE
+            engine.result(k, copy_image=False)
+    for thing in (heavy_scene, light_scene, ctx, *others):
+        thing.close()
+    # 4 MB: 0.15 ms over the link; a launch of the worker's traversal lasts milliseconds.
+    assert busy < 3.0 * idle + 0.5e-3, f"idle {1e3 * idle:.2f} ms, busy {1e3 * busy:.2f} ms"
