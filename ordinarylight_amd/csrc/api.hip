@@ -274,7 +274,7 @@ int olhip_create(int device, olhip_ctx** out) {
     OL_HIP_CHECK(hipGetDeviceProperties(&prop, device));
     ctx->cu_count = prop.multiProcessorCount;
     ctx->trace_scratch = trace_scratch_address(device);
-    ctx->copier = std::make_unique<HostCopier>(device);
+    ctx->copier = HostCopier::of(device);
     *out = ctx.release();
   });
 }

@@ -277,8 +277,8 @@ struct olhip_ctx {
   std::mutex query_mu;
   DevBuf query_o, query_d, query_h;
   float4* query_host = nullptr;  // origins, directions, hits, then the overflow word
-  // Host copies of images, products, rays and hits.
-  std::unique_ptr<HostCopier> copier;
+  // Host copies of images, products, rays and hits (the device's).
+  std::shared_ptr<HostCopier> copier;
   // Device address of the fixed traversal spill array (olhip_trace_device).
   uint32_t* trace_scratch = nullptr;
   // Reference-estimator frame.

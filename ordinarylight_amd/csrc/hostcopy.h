@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <memory>
 #include <mutex>
 #include <vector>
 
@@ -24,27 +25,35 @@
 // Pages of a fresh destination are populated by one call per part (27-66 us per
 // MB, page faults take 100-220), or beforehand where the caller knows its
 // destination while the device still works (Prefault).
-// Downloads of one HostCopier run one after the other; it holds 1.5 MB of
-// pinned memory, made at its first download.
+//
+// The contexts of a device share one HostCopier, freed with the last of them.
+// Its ring costs what it saves over some 40 MB (a stream 0.2 ms, the
+// allocation 0.1, the first touch of its pages 0.34 per MB; it saves 20 us per
+// MB), so the first kPlain bytes are copied plainly, and a context made beside
+// others finds the ring ready: with a ring of 8 MB per context, made in its
+// first frame, that frame took 1 to 4 ms longer.  One download uses the ring at
+// a time; one that finds it in use is copied plainly beside it.
 class HostCopier {
  public:
+  static std::shared_ptr<HostCopier> of(int device);
   explicit HostCopier(int device) : device_(device) {}
   ~HostCopier();
   HostCopier(const HostCopier&) = delete;
   HostCopier& operator=(const HostCopier&) = delete;
-  // Work that writes `dev` must have completed.
+  // Work that writes `dev` must have completed.  From any thread.
   void download(void* dst, const void* dev, size_t bytes);
   // Maps the pages of [dst, dst + bytes) without changing their contents.
   // A hint: what cannot be mapped this way faults page by page when written.
   static void prefault(void* dst, size_t bytes);
 
  private:
-  static constexpr size_t kPiece = size_t(768) << 10;
-
-  void prepare();
+  static constexpr size_t kPiece = size_t(768) << 10, kPlain = size_t(32) << 20;
+  bool ring_for(size_t bytes);
+  void through_ring(char* dst, const char* dev, size_t bytes);
 
   int device_;
-  std::mutex use_;  // one download at a time
+  std::mutex use_;  // the ring, and the words below
+  size_t plain_ = 0;  // bytes copied plainly before the ring was made
   hipStream_t stream_ = nullptr;
   char* ring_ = nullptr;  // two pieces
 };

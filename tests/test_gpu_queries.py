@@ -1,6 +1,6 @@
 """Ray queries and downloads at the sizes where they change their route:
-pinned buffers up to 4096 rays, flags per 256 KB, pieces of 2 MB, a ring of
-four pieces."""
+pinned buffers up to 4096 rays, plain copies until a device's contexts have
+downloaded 32 MB, then pieces of 768 KB through a ring of two."""
 
 import numpy as np
 import pytest
@@ -24,7 +24,8 @@ def scene(hip_device):
 
 
 @pytest.mark.parametrize("n", [1, 4095, 4096, 4097, (256 << 10) // RAY - 1, (256 << 10) // RAY + 1, (2 << 20) // RAY,
-                               (2 << 20) // RAY + 1, (10 << 20) // RAY + 3])
+                               (2 << 20) // RAY + 1, (10 << 20) // RAY + 3, (768 << 10) // RAY - 1, (768 << 10) // RAY,
+                               (768 << 10) // RAY + 1, 2 * (768 << 10) // RAY + 1, 3 * (768 << 10) // RAY + 1])
 def test_hits_do_not_depend_on_the_size_of_the_call(scene, n):
     rng = np.random.default_rng(n)
     o = rng.uniform(-1.0, 1.0, (n, 3)).astype(np.float32)
