@@ -113,7 +113,7 @@ Engine::Engine(olhip_ctx* ctx, const olhip_engine_config& cfg) : ctx_(ctx), cfg_
   jobs_state_.assign(kMaxJobs, JobDev{});
   for (int b = 0; b < 2; ++b) {
     stage_host_[b] = pinned<StepStage>(1);
-    report_host_[b] = pinned<uint32_t>(C_WORDS - C_OVERFLOW);
+    report_host_[b] = pinned<uint32_t>(R_WORDS);
   }
   if (cfg_.use_graph) OL_HIP_CHECK(hipStreamCreateWithFlags(&capture_, hipStreamNonBlocking));
   OL_HIP_CHECK(hipEventCreate(&begin_));
@@ -752,7 +752,7 @@ void Engine::retire_front() {
     if (f.traced) {
       ++steps_;
       const uint32_t* report = report_host_[f.report];
-      const uint32_t* rep = report + (C_REPORT - C_OVERFLOW);
+      const uint32_t* rep = report + R_JOBS;
       // The overflow flags are sticky until reset; a reset queued after an
       // overflow follows the steps already in flight, whose reports still
       // show it.  Those steps' jobs were failed with the first report.

@@ -85,10 +85,10 @@ constexpr uint32_t C_OVERFLOW = C_WS2 + kWorkStripes * kCursorStride, C_STACK = 
 // Steps traced since the counters were cleared (its parity picks the host
 // report buffer).
 constexpr uint32_t C_STEPS = C_OVERFLOW + 2;
-// Report layout (host buffers, from C_OVERFLOW on): the two overflow words,
-// then kMaxJobs x 4: rays traced, shadow rays, live paths, shaded hits.
-constexpr uint32_t C_REPORT = C_OVERFLOW + 8;
-constexpr uint32_t C_WORDS = C_REPORT + 4 * kMaxJobs;
+constexpr uint32_t C_WORDS = C_OVERFLOW + 8;
+// Report layout (host buffers): the two overflow words, then from R_JOBS on
+// kMaxJobs x 4: rays traced, shadow rays, live paths, shaded hits.
+constexpr uint32_t R_JOBS = 8, R_WORDS = R_JOBS + 4 * kMaxJobs;
 OL_HD constexpr uint32_t c_queue(uint32_t q) { return q ? C_Q1 : C_Q0; }
 OL_HD constexpr uint32_t c_groups(uint32_t p) { return p ? C_G1 : C_G0; }
 OL_HD constexpr uint32_t c_entries(uint32_t p) { return p ? C_E1 : C_E0; }

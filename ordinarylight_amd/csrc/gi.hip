@@ -51,7 +51,7 @@ constexpr uint32_t kRefillMin2 = 8;
 // filled run by run instead, a small job's single run left a thread writing
 // up to 1024 entries alone (30 us of a 250 us step of a 256 x 256 frame).
 struct PlanShared {
-  uint32_t prefix[kRuns], wave_tot[16], wave_last[16], shift;
+  uint32_t prefix[kRuns], wave_tot[16], wave_last[16];
 };
 template <bool kCapped>
 OL_DEV void plan_runs(const uint32_t* __restrict__ counts, uint32_t* __restrict__ out, uint32_t kind,
@@ -1829,7 +1829,7 @@ __global__ void __launch_bounds__(1024) k_epilogue(Wave W, uint32_t in, uint32_t
   auto report = [&](uint32_t word, uint32_t v) {
     __hip_atomic_store(&host[word], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   };
-  if (t < 4 * kMaxJobs) report(C_REPORT - C_OVERFLOW + t, sh.rep[t]);
+  if (t < 4 * kMaxJobs) report(R_JOBS + t, sh.rep[t]);
   if (t < 2u) report(t, W.ctr[C_OVERFLOW + t]);
   __syncthreads();
   if (t == 0u) ++W.ctr[C_STEPS];

@@ -42,7 +42,6 @@ OL_DEV bool ol_tri_test(f3 o, f3 d, float4 a, float4 e1, float4 e2, float& t, fl
 
 struct RayPre {
   f3 o, d, inv;
-  uint32_t neg;  // bit a set when the direction's axis-a component is negative
 };
 
 OL_DEV RayPre ray_pre(f3 o, f3 d) {
@@ -51,7 +50,6 @@ OL_DEV RayPre ray_pre(f3 o, f3 d) {
   r.o = o;
   r.d = d;
   r.inv = mk3(1.0f / safe(d.x), 1.0f / safe(d.y), 1.0f / safe(d.z));
-  r.neg = (r.inv.x < 0.0f ? 1u : 0u) | (r.inv.y < 0.0f ? 2u : 0u) | (r.inv.z < 0.0f ? 4u : 0u);
   return r;
 }
 
@@ -66,7 +64,6 @@ OL_DEV RayPre ray_pre_fast(f3 o, f3 d) {
   r.o = o;
   r.d = d;
   r.inv = mk3(__builtin_amdgcn_rcpf(safe(d.x)), __builtin_amdgcn_rcpf(safe(d.y)), __builtin_amdgcn_rcpf(safe(d.z)));
-  r.neg = (r.inv.x < 0.0f ? 1u : 0u) | (r.inv.y < 0.0f ? 2u : 0u) | (r.inv.z < 0.0f ? 4u : 0u);
   return r;
 }
 
