@@ -204,9 +204,7 @@ __global__ void __launch_bounds__(BLOCK) k_e0_trace(E0Params P, E0State S, uint3
         const float cull = bt < (U)3.0e38 ? cull_distance((float)bt) + 1e-6f : INFINITY;
         double p[4];
         const uint32_t hits = node_children<true>(w0, w1, w2, w3, rp, 0.0f, cull, p);
-        // Near to far (the last hit child first): leaves are tested at once,
-        // the nearest inner child comes next, the others go on the stack.
-        uint32_t next = OL_NONE;
+        // Leaves are tested at once, near to far (the last hit child first).
 #pragma unroll
         for (int k = 3; k >= 0; --k) {
           if ((uint32_t)k >= hits) continue;
@@ -222,13 +220,20 @@ __global__ void __launch_bounds__(BLOCK) k_e0_trace(E0Params P, E0State S, uint3
                 bi = orig;
               }
             }
-          } else if (next == OL_NONE) {
-            next = c;
-          } else if (sp < (uint32_t)STACK) {
-            col[(sp++) * BLOCK] = c;
-          } else {
-            atomicOr(&S.ctr[1], 1u);
           }
+        }
+        // The nearest inner child comes next, the others wait on the stack
+        // with the nearer ones above.
+        uint32_t next = OL_NONE;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t c = pair_word(p[k]);
+          if ((uint32_t)k >= hits || child_is_leaf(c)) continue;
+          if (next != OL_NONE) {
+            if (sp < (uint32_t)STACK) col[(sp++) * BLOCK] = next;
+            else atomicOr(&S.ctr[1], 1u);
+          }
+          next = c;
         }
         if (next != OL_NONE) {
           node = next;
