@@ -542,7 +542,7 @@ void build_top_level(olhip_scene* sc, const olhip_instanced_desc* d, hipStream_t
   // read of the leaf record.
   {
     std::vector<float4> leaves(3ull * I);
-    OL_HIP_CHECK(hipMemcpy(leaves.data(), sc->bvh.tri.ptr, sizeof(float4) * leaves.size(), hipMemcpyDeviceToHost));
+    copy_down(leaves.data(), sc->bvh.tri.ptr, sizeof(float4) * leaves.size(), s);
     std::vector<InstanceDev> ordered(I);
     for (uint32_t j = 0; j < I; ++j) {
       uint32_t k;
@@ -837,10 +837,9 @@ int olhip_scene_bvh(const olhip_scene* scene, void* nodes, void* tri) {
   return guarded([&] {
     require(scene != nullptr, "scene must not be NULL");
     OL_HIP_CHECK(hipSetDevice(scene->ctx->device));
-    OL_HIP_CHECK(hipStreamSynchronize(scene->ctx->stream));
-    if (nodes && scene->bvh.node_count) bvh_export_nodes(scene->bvh, static_cast<Node4*>(nodes));
-    if (tri && scene->tri_count)
-      OL_HIP_CHECK(hipMemcpy(tri, scene->bvh.tri.ptr, 48ull * scene->tri_count, hipMemcpyDeviceToHost));
+    hipStream_t s = scene->ctx->stream;
+    if (nodes && scene->bvh.node_count) bvh_export_nodes(scene->bvh, static_cast<Node4*>(nodes), s);
+    if (tri && scene->tri_count) copy_down(tri, scene->bvh.tri.ptr, 48ull * scene->tri_count, s);
   });
 }
 
@@ -960,7 +959,7 @@ int olhip_render_products(olhip_ctx* ctx, const olhip_scene* sc, const olhip_cam
     ctx->image_width = width;
     ctx->image_height = height;
     if (d.products) eng.products(id, depth, normal, primitive, variance);
-    if (out_rgba) ctx->copier->download(out_rgba, ctx->image.ptr, sizeof(float4) * np);
+    if (out_rgba) ctx->download(out_rgba, ctx->image.ptr, sizeof(float4) * np);
     eng.take_result(id, nullptr, &js);
     if (stats_out) {
       olhip_stats& o = *stats_out;
@@ -1112,7 +1111,7 @@ int olhip_frame_download(olhip_ctx* ctx, float* out_rgba) {
     require(ctx->image_pixels > 0, "no frame has been rendered");
     OL_HIP_CHECK(hipSetDevice(ctx->device));
     OL_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-    ctx->copier->download(out_rgba, ctx->image.ptr, sizeof(float4) * ctx->image_pixels);
+    ctx->download(out_rgba, ctx->image.ptr, sizeof(float4) * ctx->image_pixels);
   });
 }
 
@@ -1142,7 +1141,7 @@ int olhip_frame_output(olhip_ctx* ctx, uint32_t format, float exposure, uint32_t
                   s);
     OL_HIP_CHECK(hipGetLastError());
     OL_HIP_CHECK(hipStreamSynchronize(s));
-    if (!out_on_device) ctx->copier->download(out, staging.ptr, bytes);
+    if (!out_on_device) ctx->download(out, staging.ptr, bytes);
   });
 }
 
@@ -1193,7 +1192,7 @@ struct QueryBuffers {
   }
   void get(float* to, const float4* from) {
     if (direct) std::memcpy(to, from, sizeof(float4) * (size_t)n);
-    else ctx->copier->download(to, from, sizeof(float4) * (size_t)n);
+    else ctx->download(to, from, sizeof(float4) * (size_t)n);
   }
 };
 
@@ -1399,7 +1398,7 @@ int olhip_e0_trace(olhip_ctx* ctx, uint32_t* n_hit, uint32_t* n_active) {
     OL_HIP_CHECK(hipGetLastError());
     f.n_hit = e0_compact(f.state, f.n_active, s);
     uint32_t ctr[4];
-    OL_HIP_CHECK(hipMemcpy(ctr, f.ctr.ptr, 16, hipMemcpyDeviceToHost));
+    copy_down(ctr, f.ctr.ptr, 16, s);
     if (ctr[1]) throw OlError{OLHIP_ERR_RUNTIME, "traversal stack overflow"};
     *n_hit = f.n_hit;
   });
@@ -1410,8 +1409,7 @@ int olhip_e0_last_hits(olhip_ctx* ctx, int32_t* tri, uint32_t n_active) {
     require(ctx && tri, "arguments must not be NULL");
     auto& f = ctx->e0;
     require(n_active <= f.params.width * f.params.height, "n_active too large");
-    OL_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-    if (n_active) OL_HIP_CHECK(hipMemcpy(tri, f.htri.ptr, 4ull * n_active, hipMemcpyDeviceToHost));
+    if (n_active) copy_down(tri, f.htri.ptr, 4ull * n_active, ctx->stream);
   });
 }
 
@@ -1455,7 +1453,7 @@ int olhip_e0_end(olhip_ctx* ctx, uint32_t samples, float* out_rgba) {
     e0_finish(f.params, f.state, samples, f.out.as<float4>(), s);
     OL_HIP_CHECK(hipGetLastError());
     OL_HIP_CHECK(hipStreamSynchronize(s));
-    ctx->copier->download(out_rgba, f.out.ptr, 16ull * f.params.width * f.params.height);
+    ctx->download(out_rgba, f.out.ptr, 16ull * f.params.width * f.params.height);
     f.open = false;
   });
 }

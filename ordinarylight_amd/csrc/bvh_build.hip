@@ -595,11 +595,11 @@ void build_nodes(const BvhInput& in, const BvhTopology& tp, BvhOutput& out, hipS
 
 }  // namespace
 
-void bvh_export_nodes(const BvhOutput& built, Node4* out) {
+void bvh_export_nodes(const BvhOutput& built, Node4* out, hipStream_t stream) {
   const uint32_t n = built.node_count;
   std::vector<WideNode> nodes(n);
   if (n == 0) return;
-  OL_HIP_CHECK(hipMemcpy(nodes.data(), built.nodes.ptr, sizeof(WideNode) * (size_t)n, hipMemcpyDeviceToHost));
+  copy_down(nodes.data(), built.nodes.ptr, sizeof(WideNode) * (size_t)n, stream);
   auto exponent = [](float scale) {
     uint32_t bits;
     std::memcpy(&bits, &scale, sizeof(bits));

@@ -135,6 +135,7 @@ Engine::~Engine() {
   stop_worker();
   (void)hipSetDevice(ctx_->device);
   (void)hipStreamSynchronize(ctx_->stream);
+  ctx_->steps_queued -= (uint32_t)inflight_.size();
   // Jobs never taken leave their buffers to the context's pool.
   for (auto& kv : jobs_) keep_buffers(*kv.second);
   for (auto& kv : graphs_) (void)hipGraphExecDestroy(kv.second);
@@ -234,8 +235,7 @@ void Engine::set_work_counters(bool on) {
 }
 
 void Engine::read_work(unsigned long long out[kWorkWords]) {
-  OL_HIP_CHECK(hipStreamSynchronize(ctx_->stream));
-  OL_HIP_CHECK(hipMemcpy(out, work_.ptr, 8 * kWorkWords, hipMemcpyDeviceToHost));
+  copy_down(out, work_.ptr, 8 * kWorkWords, ctx_->stream);
 }
 
 uint64_t Engine::submit(const olhip_job_desc& d) {
@@ -553,6 +553,7 @@ uint32_t Engine::step() {
   } catch (...) {
     // The queued steps' reports can no longer be matched to jobs.
     (void)hipStreamSynchronize(ctx_->stream);
+    ctx_->steps_queued -= (uint32_t)inflight_.size();
     inflight_.clear();
     inflight_count_ = 0;
     throw;
@@ -716,6 +717,7 @@ bool Engine::launch_next() {
   }
   ++seq_;
   inflight_.push_back(std::move(f));
+  ++ctx_->steps_queued;
   return true;
 }
 
@@ -726,7 +728,9 @@ bool Engine::launch_next() {
 void Engine::retire_front() {
   InFlight f = std::move(inflight_.front());
   inflight_.pop_front();
-  OL_HIP_CHECK(hipEventSynchronize(f.done));
+  const hipError_t done = hipEventSynchronize(f.done);
+  --ctx_->steps_queued;
+  OL_HIP_CHECK(done);
   float step_ms = 0.0f;
   OL_HIP_CHECK(hipEventElapsedTime(&step_ms, f.begin, f.done));
   if (f.timed) {
@@ -872,7 +876,7 @@ void Engine::take_result(uint64_t id, float* out_rgba, olhip_job_stats* stats) {
   }
   OL_HIP_CHECK(hipSetDevice(ctx_->device));
   if (out_rgba)
-    ctx_->copier->download(out_rgba, j->image.ptr, sizeof(float4) * j->desc.width * j->desc.height);
+    ctx_->download(out_rgba, j->image.ptr, sizeof(float4) * j->desc.width * j->desc.height);
   std::lock_guard<std::mutex> g(mu_);
   keep_buffers(*j);
 }
@@ -902,10 +906,10 @@ void Engine::products(uint64_t id, float* depth, float* normal, uint32_t* primit
   } reading{*this, *j};
   OL_HIP_CHECK(hipSetDevice(ctx_->device));
   const size_t plane = sizeof(float) * j->desc.width * j->desc.height;
-  if (depth) ctx_->copier->download(depth, j->depth.ptr, plane);
-  if (normal) ctx_->copier->download(normal, j->normal.ptr, 3 * plane);
-  if (primitive) ctx_->copier->download(primitive, j->prim.ptr, plane);
-  if (variance) ctx_->copier->download(variance, j->variance.ptr, plane);
+  if (depth) ctx_->download(depth, j->depth.ptr, plane);
+  if (normal) ctx_->download(normal, j->normal.ptr, 3 * plane);
+  if (primitive) ctx_->download(primitive, j->prim.ptr, plane);
+  if (variance) ctx_->download(variance, j->variance.ptr, plane);
 }
 
 void Engine::engine_stats(olhip_engine_stats* out) {
@@ -917,6 +921,7 @@ void Engine::start_worker() {
   if (worker_running_) return;
   stop_ = false;
   worker_running_ = true;
+  ++ctx_->workers;
   worker_ = std::thread([this] {
     (void)hipSetDevice(ctx_->device);
     while (true) {
@@ -959,4 +964,5 @@ void Engine::stop_worker() {
   }
   worker_.join();
   worker_running_ = false;
+  --ctx_->workers;
 }

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <condition_variable>
 #include <cstddef>
 #include <memory>
 #include <mutex>
@@ -16,8 +17,8 @@
 // 1.8), but its blocks wait for room beside a worker's traversal waves, which
 // live as long as their launch: a 1 MB image fetched beside a rendering worker
 // took 0.7 ms at the median and 11 ms at worst, here 0.1 and 0.2.
-// Pieces are awaited by synchronising the ring's stream, which follows the
-// copy itself.  An event would go through the stream's hardware queue, which
+// Pieces are awaited by synchronising their stream, which follows the copy
+// itself.  An event would go through the stream's hardware queue, which
 // may be the one that a worker's steps use (there are four per process): each
 // piece then waited for a step, 33 MB for 130 ms.
 // Two pieces of 768 KB: 5 MB in 0.17 ms, 33 MB in 1.40 ms into mapped pages
@@ -26,36 +27,44 @@
 // MB, page faults take 100-220), or beforehand where the caller knows its
 // destination while the device still works (Prefault).
 //
-// The contexts of a device share one HostCopier, freed with the last of them.
-// Its ring costs what it saves over some 40 MB (a stream 0.2 ms, the
-// allocation 0.1, the first touch of its pages 0.34 per MB; it saves 20 us per
-// MB), so the first kPlain bytes are copied plainly, and a context made beside
-// others finds the ring ready: with a ring of 8 MB per context, made in its
-// first frame, that frame took 1 to 4 ms longer.  One download uses the ring at
-// a time; one that finds it in use is copied plainly beside it.
+// The contexts of a device share one HostCopier, freed with the last of them: a
+// context made beside others finds a ring ready.  (With 8 MB of its own, made
+// in its first frame, that frame took 1 to 4 ms longer; the first touch of
+// pinned pages is the dearest, 0.34 ms per MB.)  A second ring is made when the
+// first is in use, up to kRings; further downloads wait for one.
 class HostCopier {
  public:
   static std::shared_ptr<HostCopier> of(int device);
-  explicit HostCopier(int device) : device_(device) {}
-  ~HostCopier();
+  explicit HostCopier(int device) : device_(device) { idle_.reserve(kRings); }
+  ~HostCopier() { (void)hipSetDevice(device_); }
   HostCopier(const HostCopier&) = delete;
   HostCopier& operator=(const HostCopier&) = delete;
-  // Work that writes `dev` must have completed.  From any thread.
-  void download(void* dst, const void* dev, size_t bytes);
+  // Work that writes `dev` must have completed.  From any thread.  `idle`: a
+  // stream that nothing else uses meanwhile; without one the copy runs on a
+  // stream of the ring's, made when it is first needed (0.25 ms, 3.5 ms while
+  // the process has hardware queues left to open).
+  void download(void* dst, const void* dev, size_t bytes, hipStream_t idle);
   // Maps the pages of [dst, dst + bytes) without changing their contents.
   // A hint: what cannot be mapped this way faults page by page when written.
   static void prefault(void* dst, size_t bytes);
 
  private:
-  static constexpr size_t kPiece = size_t(768) << 10, kPlain = size_t(32) << 20;
-  bool ring_for(size_t bytes);
-  void through_ring(char* dst, const char* dev, size_t bytes);
+  static constexpr size_t kPiece = size_t(768) << 10, kRings = 4;
+  struct Ring {
+    char* slots = nullptr;  // two pieces
+    hipStream_t stream = nullptr;
+    Ring();
+    ~Ring();
+  };
+  std::unique_ptr<Ring> take();
+  void give_back(std::unique_ptr<Ring> ring);
+  static void through(char* slots, hipStream_t stream, char* dst, const char* dev, size_t bytes);
 
   int device_;
-  std::mutex use_;  // the ring, and the words below
-  size_t plain_ = 0;  // bytes copied plainly before the ring was made
-  hipStream_t stream_ = nullptr;
-  char* ring_ = nullptr;  // two pieces
+  std::mutex mu_;
+  std::condition_variable returned_;
+  std::vector<std::unique_ptr<Ring>> idle_;
+  size_t made_ = 0;  // idle and in use
 };
 
 // Populates destinations piece by piece while their data is being computed.

@@ -11,13 +11,6 @@
 
 #include "internal.h"
 
-HostCopier::~HostCopier() {
-  (void)hipSetDevice(device_);
-  if (stream_) (void)hipStreamSynchronize(stream_);
-  if (ring_) (void)hipHostFree(ring_);
-  if (stream_) (void)hipStreamDestroy(stream_);
-}
-
 std::shared_ptr<HostCopier> HostCopier::of(int device) {
   static std::mutex mu;
   static auto& copiers = *new std::map<int, std::weak_ptr<HostCopier>>;
@@ -27,21 +20,44 @@ std::shared_ptr<HostCopier> HostCopier::of(int device) {
   return c;
 }
 
-// Whether the ring serves this download, with `use_` held.  Without pinned
-// memory for it the plain copies go on.
-bool HostCopier::ring_for(size_t bytes) {
-  if (ring_) return true;
-  if (plain_ < kPlain) {
-    plain_ += bytes;
-    return false;
+HostCopier::Ring::Ring() {
+  OL_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&slots), 2 * kPiece, hipHostMallocDefault));
+}
+
+HostCopier::Ring::~Ring() {
+  (void)hipHostFree(slots);
+  if (stream) (void)hipStreamDestroy(stream);
+}
+
+std::unique_ptr<HostCopier::Ring> HostCopier::take() {
+  {
+    std::unique_lock<std::mutex> g(mu_);
+    returned_.wait(g, [&] { return !idle_.empty() || made_ < kRings; });
+    if (!idle_.empty()) {
+      std::unique_ptr<Ring> ring = std::move(idle_.back());
+      idle_.pop_back();
+      return ring;
+    }
+    ++made_;
   }
-  plain_ = 0;
-  if (!stream_) OL_HIP_CHECK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
-  if (hipHostMalloc(reinterpret_cast<void**>(&ring_), 2 * kPiece, hipHostMallocDefault) != hipSuccess) {
-    (void)hipGetLastError();
-    ring_ = nullptr;
+  try {
+    return std::make_unique<Ring>();
+  } catch (...) {
+    {
+      std::lock_guard<std::mutex> g(mu_);
+      --made_;
+    }
+    returned_.notify_one();
+    throw;
   }
-  return ring_ != nullptr;
+}
+
+void HostCopier::give_back(std::unique_ptr<Ring> ring) {
+  {
+    std::lock_guard<std::mutex> g(mu_);
+    idle_.push_back(std::move(ring));
+  }
+  returned_.notify_one();
 }
 
 void HostCopier::prefault(void* dst, size_t bytes) {
@@ -54,30 +70,38 @@ void HostCopier::prefault(void* dst, size_t bytes) {
   if (bytes >= 4 * page) (void)madvise(reinterpret_cast<void*>(first), last - first, MADV_POPULATE_WRITE);
 }
 
-void HostCopier::download(void* dst, const void* dev, size_t bytes) {
+void HostCopier::download(void* dst, const void* dev, size_t bytes, hipStream_t idle) {
   if (bytes == 0) return;
   OL_HIP_CHECK(hipSetDevice(device_));
-  {
-    std::unique_lock<std::mutex> use(use_, std::try_to_lock);
-    if (use.owns_lock() && ring_for(bytes)) return through_ring(static_cast<char*>(dst), static_cast<const char*>(dev), bytes);
+  struct Lease {
+    HostCopier& copier;
+    std::unique_ptr<Ring> ring;
+    ~Lease() { copier.give_back(std::move(ring)); }
+  } lease{*this, take()};
+  Ring& ring = *lease.ring;
+  if (!idle && !ring.stream) OL_HIP_CHECK(hipStreamCreateWithFlags(&ring.stream, hipStreamNonBlocking));
+  const hipStream_t stream = idle ? idle : ring.stream;
+  try {
+    through(ring.slots, stream, static_cast<char*>(dst), static_cast<const char*>(dev), bytes);
+  } catch (...) {
+    (void)hipStreamSynchronize(stream);  // a piece may still be on its way into the ring
+    throw;
   }
-  prefault(dst, bytes);
-  OL_HIP_CHECK(hipMemcpy(dst, dev, bytes, hipMemcpyDeviceToHost));
 }
 
-void HostCopier::through_ring(char* dst, const char* dev, size_t bytes) {
+void HostCopier::through(char* slots, hipStream_t stream, char* dst, const char* dev, size_t bytes) {
   const size_t pieces = (bytes + kPiece - 1) / kPiece;
   auto length = [&](size_t k) { return std::min(kPiece, bytes - k * kPiece); };
-  auto slot = [&](size_t k) { return ring_ + (k & 1u) * kPiece; };
+  auto slot = [&](size_t k) { return slots + (k & 1u) * kPiece; };
   auto issue = [&](size_t k) {
-    OL_HIP_CHECK(hipMemcpyAsync(slot(k), dev + k * kPiece, length(k), hipMemcpyDeviceToHost, stream_));
+    OL_HIP_CHECK(hipMemcpyAsync(slot(k), dev + k * kPiece, length(k), hipMemcpyDeviceToHost, stream));
   };
   issue(0);
   for (size_t k = 0; k < pieces; ++k) {
     char* to = dst + k * kPiece;
     constexpr size_t part = size_t(256) << 10;
     for (size_t at = 0; at < length(k); at += part) prefault(to + at, std::min(part, length(k) - at));
-    OL_HIP_CHECK(hipStreamSynchronize(stream_));
+    OL_HIP_CHECK(hipStreamSynchronize(stream));
     if (k + 1 < pieces) issue(k + 1);
     std::memcpy(to, slot(k), length(k));
   }

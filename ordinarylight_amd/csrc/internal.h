@@ -23,6 +23,14 @@ struct OlError {
       throw OlError{-4, std::string(#expr) + ": " + hipGetErrorString(_e)};       \
   } while (0)
 
+// A small result to host memory, complete on return, after the work queued on
+// `stream`.  Never hipMemcpy: the legacy stream that it uses refuses to work
+// while another thread captures a step.
+inline void copy_down(void* dst, const void* src, size_t bytes, hipStream_t stream) {
+  OL_HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
+  OL_HIP_CHECK(hipStreamSynchronize(stream));
+}
+
 // Device buffer owned by RAII.
 struct DevBuf {
   void* ptr = nullptr;
@@ -123,7 +131,7 @@ void sah_topology(const float* box, uint32_t n, std::vector<uint32_t>& order, st
 void bvh_build(const BvhInput& in, BvhOutput& out, hipStream_t stream, bool keep_topology = false);
 // The built nodes in their exported form: numbered breadth-first, exponents
 // packed, missing children marked (node_count records).
-void bvh_export_nodes(const BvhOutput& built, Node4* out);
+void bvh_export_nodes(const BvhOutput& built, Node4* out, hipStream_t stream);
 // Recomputes the boxes, the wide nodes and the leaf triangles of a kept
 // topology for new vertex positions (same triangles, same indices), as an
 // acceleration-structure update does: the leaf order stays, boxes follow the

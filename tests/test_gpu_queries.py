@@ -1,6 +1,5 @@
 """Ray queries and downloads at the sizes where they change their route:
-pinned buffers up to 4096 rays, plain copies until a device's contexts have
-downloaded 32 MB, then pieces of 768 KB through a ring of two."""
+pinned buffers up to 4096 rays, then pieces of 768 KB through a ring of two."""
 
 import numpy as np
 import pytest
