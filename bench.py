@@ -144,7 +144,7 @@ def roofline_of(kernel, bytes_per_launch, avg_ms, traffic, traffic_source):
     achieved = bytes_per_launch / (avg_ms * 1e-3) / 1e9
     out = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
            "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "kernel": kernel,
-           "basis": "algorithmic bytes per launch / average launch time",
+           "basis": "algorithmic bytes per launch (mostly cache hits; `traffic` leaves the L2) / average launch time",
            "avg_launch_ms": round(avg_ms, 4), "bytes_per_launch": int(bytes_per_launch),
            "traffic_source": traffic_source if traffic is not None else None}
     if traffic is not None:

@@ -319,7 +319,7 @@ typedef struct olhip_engine_stats {
   uint32_t resident_jobs, queued_jobs, max_resident_jobs;
   uint32_t fused_steps;  /* steps run as one traversal-and-shading kernel (hybrid strategy) */
   uint64_t path_slots, entry_slots;
-  double device_ms;  /* stream time of the retired steps, first launch to report copy */
+  double device_ms;  /* stream time of the retired steps; a step queued behind another starts at its end */
 } olhip_engine_stats;
 
 int olhip_engine_create(olhip_ctx* ctx, const olhip_engine_config* config, olhip_engine** out);
@@ -366,7 +366,7 @@ int olhip_set_profiling(olhip_ctx* ctx, int enabled);
 /* Count traversal work (nodes visited, triangles tested) in olhip_stats. */
 int olhip_set_work_counters(olhip_ctx* ctx, int enabled);
 /* Traversal launch shape: stack entries kept in LDS per lane (the rest of
- * the 3 * depth + 1 entries spill to a global per-lane column) and the block
+ * the 3 * depth + 2 entries spill to a global per-lane column) and the block
  * size.  Supported: (8|12|24|32|48, 128) and (16, 64|128|256).  Results do
  * not depend on these settings. */
 int olhip_set_traversal(olhip_ctx* ctx, int lds_entries, int block);
