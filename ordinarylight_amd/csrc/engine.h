@@ -279,12 +279,8 @@ struct olhip_ctx {
   float4* query_host = nullptr;  // origins, directions, hits, then the overflow word
   // Host copies of images, products, rays and hits (the device's).
   std::shared_ptr<HostCopier> copier;
-  // Steps that the context's engines have queued, and their running workers.
-  // Beside either a download keeps off the context's stream, where each of its
-  // pieces would wait for a step.
-  std::atomic<uint32_t> steps_queued{0}, workers{0};
   void download(void* dst, const void* dev, size_t bytes) {
-    copier->download(dst, dev, bytes, steps_queued || workers ? nullptr : stream);
+    copier->download(dst, dev, bytes, copier->device_busy() ? nullptr : stream);
   }
   // Device address of the fixed traversal spill array (olhip_trace_device).
   uint32_t* trace_scratch = nullptr;

@@ -135,7 +135,7 @@ Engine::~Engine() {
   stop_worker();
   (void)hipSetDevice(ctx_->device);
   (void)hipStreamSynchronize(ctx_->stream);
-  ctx_->steps_queued -= (uint32_t)inflight_.size();
+  ctx_->copier->steps_queued -= (uint32_t)inflight_.size();
   // Jobs never taken leave their buffers to the context's pool.
   for (auto& kv : jobs_) keep_buffers(*kv.second);
   for (auto& kv : graphs_) (void)hipGraphExecDestroy(kv.second);
@@ -553,7 +553,7 @@ uint32_t Engine::step() {
   } catch (...) {
     // The queued steps' reports can no longer be matched to jobs.
     (void)hipStreamSynchronize(ctx_->stream);
-    ctx_->steps_queued -= (uint32_t)inflight_.size();
+    ctx_->copier->steps_queued -= (uint32_t)inflight_.size();
     inflight_.clear();
     inflight_count_ = 0;
     throw;
@@ -717,7 +717,7 @@ bool Engine::launch_next() {
   }
   ++seq_;
   inflight_.push_back(std::move(f));
-  ++ctx_->steps_queued;
+  ++ctx_->copier->steps_queued;
   return true;
 }
 
@@ -729,7 +729,7 @@ void Engine::retire_front() {
   InFlight f = std::move(inflight_.front());
   inflight_.pop_front();
   const hipError_t done = hipEventSynchronize(f.done);
-  --ctx_->steps_queued;
+  --ctx_->copier->steps_queued;
   OL_HIP_CHECK(done);
   float step_ms = 0.0f;
   OL_HIP_CHECK(hipEventElapsedTime(&step_ms, f.begin, f.done));
@@ -921,7 +921,7 @@ void Engine::start_worker() {
   if (worker_running_) return;
   stop_ = false;
   worker_running_ = true;
-  ++ctx_->workers;
+  ++ctx_->copier->workers;
   worker_ = std::thread([this] {
     (void)hipSetDevice(ctx_->device);
     while (true) {
@@ -964,5 +964,5 @@ void Engine::stop_worker() {
   }
   worker_.join();
   worker_running_ = false;
-  --ctx_->workers;
+  --ctx_->copier->workers;
 }

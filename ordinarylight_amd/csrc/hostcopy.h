@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <condition_variable>
 #include <cstddef>
 #include <memory>
@@ -23,6 +24,10 @@
 // piece then waited for a step, 33 MB for 130 ms.
 // Two pieces of 768 KB: 5 MB in 0.17 ms, 33 MB in 1.40 ms into mapped pages
 // and 1.94 into fresh ones; 256 KB 0.26, 1.66 and 2.54, 1 MB 0.21, 1.29 and 2.39.
+// The driver wipes freed device memory with the same engine: for some tens of
+// milliseconds after 1 GB has been freed a piece takes 145 us instead of 22.
+// Where a piece is that late and the device is idle, a kernel brings the rest
+// (26 us a piece; 33 MB in 2.2 ms instead of 4.7).
 // Pages of a fresh destination are populated by one call per part (27-66 us per
 // MB, page faults take 100-220), or beforehand where the caller knows its
 // destination while the device still works (Prefault).
@@ -40,10 +45,16 @@ class HostCopier {
   HostCopier(const HostCopier&) = delete;
   HostCopier& operator=(const HostCopier&) = delete;
   // Work that writes `dev` must have completed.  From any thread.  `idle`: a
-  // stream that nothing else uses meanwhile; without one the copy runs on a
-  // stream of the ring's, made when it is first needed (0.25 ms, 3.5 ms while
-  // the process has hardware queues left to open).
+  // stream that nothing else uses meanwhile, on a device with nothing else to
+  // do; without one the copy runs on a stream of the ring's, made when it is
+  // first needed (0.25 ms, 3.5 ms while the process has hardware queues left
+  // to open).
   void download(void* dst, const void* dev, size_t bytes, hipStream_t idle);
+  // Steps that the device's engines have queued, and their running workers.
+  // Beside either a download keeps off its context's stream, where each piece
+  // would wait for a step, and off the compute units.
+  std::atomic<uint32_t> steps_queued{0}, workers{0};
+  bool device_busy() const { return steps_queued != 0 || workers != 0; }
   // Maps the pages of [dst, dst + bytes) without changing their contents.
   // A hint: what cannot be mapped this way faults page by page when written.
   static void prefault(void* dst, size_t bytes);
@@ -58,7 +69,7 @@ class HostCopier {
   };
   std::unique_ptr<Ring> take();
   void give_back(std::unique_ptr<Ring> ring);
-  static void through(char* slots, hipStream_t stream, char* dst, const char* dev, size_t bytes);
+  static void through(char* slots, hipStream_t stream, bool idle, char* dst, const char* dev, size_t bytes);
 
   int device_;
   std::mutex mu_;
